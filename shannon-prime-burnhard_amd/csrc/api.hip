@@ -200,9 +200,16 @@ size_t q8_planes_bytes(int T, int nb) {
     return (((size_t)T * nb * (256 + Q8MN_BYTES + 32 + 4)) + 255) & ~(size_t)255;
 }
 
+// The RMS norm of a matmul's input rows (weights w, eps), applied by the pass
+// that quantises them.
+struct Norm {
+    const float* w;
+    float eps;
+};
+
 // extra: bytes of scratch wanted behind the planes (at q8_planes_bytes)
 int q8_planes(spq4k_ctx* c, const float* x, int64_t x_tstride, int T, int nb, Q8Planes* Q, bool perm = false,
-              size_t extra = 0) {
+              size_t extra = 0, const Norm* norm = nullptr) {
     const size_t items = (size_t)T * nb;
     int rc = ensure_scratch(c, q8_planes_bytes(T, nb) + extra);
     if (rc) return rc;
@@ -210,7 +217,8 @@ int q8_planes(spq4k_ctx* c, const float* x, int64_t x_tstride, int T, int nb, Q8
     uint8_t* mn = c->scratch + items * 256;
     int16_t* bs = (int16_t*)(c->scratch + items * (256 + Q8MN_BYTES));
     float* d = (float*)(c->scratch + items * (256 + Q8MN_BYTES + 32));
-    hipError_t e = launch_quantize_q8k_planes(x, x_tstride, T, nb, qs, bs, d, mn, perm, c->stream);
+    hipError_t e = norm ? launch_rms_norm_planes(x, x_tstride, T, nb, norm->w, norm->eps, qs, bs, d, mn, perm, c->stream)
+                        : launch_quantize_q8k_planes(x, x_tstride, T, nb, qs, bs, d, mn, perm, c->stream);
     if (e != hipSuccess) return hip_fail(c, e, "quantize_q8k_planes launch");
     Q->qs = qs;
     Q->bs = bs;
@@ -301,7 +309,7 @@ DecodeCfg plan_decode(const spq4k_ctx* c, int fmt, int nb_rows, int64_t rows, bo
 }
 
 int gemm_segments(spq4k_ctx* c, int n, const spq4k_weights* const* W, const float* X, float* const* Y, int64_t T,
-                  int mode);
+                  int mode, const Norm* norm = nullptr);
 
 // A fusion asked of gemv_launch: the decode kernel's RMS-norm prologue
 // (norm_w) and / or its gate-up SiLU epilogue (glu: W[0] gate, W[1] up, y[0]
@@ -466,8 +474,9 @@ int q80_dense(spq4k_ctx* c, int n, const spq4k_weights* const* W, const float* X
     return 0;
 }
 
+// norm (K-quant weights, T > 1): x is normalised as its planes are made.
 int gemv_launch(spq4k_ctx* c, int n, const spq4k_weights* const* W, const float* x, float* const* y, int64_t T,
-                const Fuse* fuse = nullptr) {
+                const Fuse* fuse = nullptr, const Norm* norm = nullptr) {
     if (n < 1 || n > GEMV_MAX_SEG) return set_err(c, -EINVAL, "gemv: n=%d matrices (1..4)", n);
     if (T < 1 || T > SPQ4K_GEMV_MAX_T) return set_err(c, -EINVAL, "gemv: T=%lld (1..8)", (long long)T);
     if (!x || !aligned(x, 16)) return set_err(c, -EINVAL, "gemv: x null or not 16-byte aligned");
@@ -552,7 +561,7 @@ int gemv_launch(spq4k_ctx* c, int n, const spq4k_weights* const* W, const float*
         !(p.fmt != WF_Q4K && c->gemm_mode == 1)) {
         // 4 <= T <= 8: the sdot4 kernel's integer work grows with T while the
         // matrix cores' 16-token tile costs the same from T = 1 to 16
-        return gemm_segments(c, n, W, x, y, T, c->gemm_mode == 1 ? 1 : 0);
+        return gemm_segments(c, n, W, x, y, T, c->gemm_mode == 1 ? 1 : 0, norm);
     }
     const int cb_max = LDS_BUDGET / ((int)T * 292);
     p.chunk_blocks = p.nb < cb_max ? p.nb : cb_max;
@@ -561,8 +570,9 @@ int gemv_launch(spq4k_ctx* c, int n, const spq4k_weights* const* W, const float*
     bool preq = (int64_t)p.nb * T > 48;
     if (c->preq_mode == 1) preq = true;
     if (c->preq_mode == 2) preq = false;
+    if (norm) preq = true;
     if (preq) {
-        int rc = q8_planes(c, x, K, (int)T, p.nb, &p.Q);
+        int rc = q8_planes(c, x, K, (int)T, p.nb, &p.Q, false, 0, norm);
         if (rc) return rc;
     }
     hipError_t e = launch_gemv(p, (int)T, bpr, (int)tiles, c->stream);
@@ -573,7 +583,8 @@ int gemv_launch(spq4k_ctx* c, int n, const spq4k_weights* const* W, const float*
 // Batches of more than SPQ4K_GEMV_MAX_T tokens for formats without a
 // matrix-core kernel (Q6_K): X is quantised once into Q8_K planes, then the
 // sdot4 GEMV runs over slices of 8 tokens of those planes.
-int gemv_chunked(spq4k_ctx* c, int n, const spq4k_weights* const* W, const float* X, float* const* Y, int64_t T) {
+int gemv_chunked(spq4k_ctx* c, int n, const spq4k_weights* const* W, const float* X, float* const* Y, int64_t T,
+                 const Norm* norm) {
     const int64_t K = W[0]->K;
     const int nb = (int)(K / SPQ4K_QK_K);
     int64_t Ms[GEMV_MAX_SEG];
@@ -606,7 +617,7 @@ int gemv_chunked(spq4k_ctx* c, int n, const spq4k_weights* const* W, const float
     const int cb_max = LDS_BUDGET / (SPQ4K_GEMV_MAX_T * 292);
     p.chunk_blocks = nb < cb_max ? nb : cb_max;
     Q8Planes Q;
-    int rc = q8_planes(c, X, K, (int)T, nb, &Q);
+    int rc = q8_planes(c, X, K, (int)T, nb, &Q, false, 0, norm);
     if (rc) return rc;
     for (int64_t t0 = 0; t0 < T; t0 += SPQ4K_GEMV_MAX_T) {
         const int tc = (int)(T - t0 < SPQ4K_GEMV_MAX_T ? T - t0 : SPQ4K_GEMV_MAX_T);
@@ -1202,7 +1213,7 @@ namespace {
 // callers): plan, quantise X once into the context scratch (with the partial
 // plane of a K split behind it), launch.
 int gemm_segments(spq4k_ctx* c, int n, const spq4k_weights* const* W, const float* X, float* const* Y, int64_t T,
-                  int mode) {
+                  int mode, const Norm* norm) {
     if (W[0]->fmt == WF_Q80) return q80_dense(c, n, W, X, Y, T);
     const int64_t K = W[0]->K;
     GemmParams p;
@@ -1228,12 +1239,12 @@ int gemm_segments(spq4k_ctx* c, int n, const spq4k_weights* const* W, const floa
     if (tiles16 * ((T + 15) / 16) > (1ll << 31) - 1 || rows > (1ll << 31) - 1)
         return set_err(c, -EINVAL, "gemm: grid too large");
     if (!fmt_has_mfma(p.fmt) || (p.fmt != WF_Q4K && mode == 1)) {   // sdot4 kernels over 8-token slices
-        if (T <= SPQ4K_GEMV_MAX_T) return gemv_launch(c, n, W, X, Y, T);
-        return gemv_chunked(c, n, W, X, Y, T);
+        if (T <= SPQ4K_GEMV_MAX_T) return gemv_launch(c, n, W, X, Y, T, nullptr, norm);
+        return gemv_chunked(c, n, W, X, Y, T, norm);
     }
     hipError_t e;
     if (gemm_use_skinny((int)T, mode)) {
-        int rc = q8_planes(c, X, K, (int)T, p.nb, &p.Q);
+        int rc = q8_planes(c, X, K, (int)T, p.nb, &p.Q, false, 0, norm);
         if (rc) return rc;
         p.total_tiles = (int32_t)tiles16;
         e = launch_gemm_skinny(p, c->stream);
@@ -1245,7 +1256,7 @@ int gemm_segments(spq4k_ctx* c, int n, const spq4k_weights* const* W, const floa
     p.cfg = g.cfg;
     p.ksplit = g.ksplit;
     p.kchunk = g.kchunk;
-    int rc = q8_planes(c, X, K, (int)T, p.nb, &p.Q, g.perm, g.partial_bytes);
+    int rc = q8_planes(c, X, K, (int)T, p.nb, &p.Q, g.perm, g.partial_bytes, norm);
     if (rc) return rc;
     p.P = g.ksplit > 1 ? reinterpret_cast<float*>(c->scratch + planes) : nullptr;
     e = launch_gemm(p, c->stream);
@@ -1476,9 +1487,17 @@ int spq4k_swiglu(spq4k_ctx* c, const float* g, const float* u, float* y, int64_t
 namespace {
 
 // matmul of n matrices sharing X, any T (spq4k_mul_mat's dispatch)
-int mul_mat_n(spq4k_ctx* c, int n, const spq4k_weights* const* W, const float* X, float* const* Y, int64_t T) {
-    if (T <= SPQ4K_GEMV_MAX_T) return gemv_launch(c, n, W, X, Y, T);
-    return gemm_segments(c, n, W, X, Y, T, c->gemm_mode);
+int mul_mat_n(spq4k_ctx* c, int n, const spq4k_weights* const* W, const float* X, float* const* Y, int64_t T,
+              const Norm* norm = nullptr) {
+    if (T <= SPQ4K_GEMV_MAX_T) return gemv_launch(c, n, W, X, Y, T, nullptr, norm);
+    return gemm_segments(c, n, W, X, Y, T, c->gemm_mode, norm);
+}
+
+// Whether a batch's norm runs in the pass that makes the activation planes:
+// K-quant weights (every path of theirs above one token reads Q8_K planes).
+// Q8_0 batches and one token outside the decode kernel keep the norm pass.
+bool norm_in_planes(const spq4k_ctx* c, const spq4k_weights* W, int64_t T) {
+    return T > 1 && W->fmt != WF_Q80 && c->preq_mode != 2;
 }
 
 int check_fused_args(spq4k_ctx* c, const char* what, int n, const spq4k_weights* const* W, const float* x,
@@ -1514,6 +1533,10 @@ int spq4k_mul_mat_rms_norm(spq4k_ctx* c, int n, const spq4k_weights* const* W, c
         rc = gemv_launch(c, n, W, x, y, T, &f);
         if (rc <= 0) return rc;
     }
+    if (norm_in_planes(c, W[0], T)) {
+        const Norm nm = {norm_w, eps};
+        return mul_mat_n(c, n, W, x, y, T, &nm);
+    }
     // unfused: the normalised rows, then the matmul on them
     const int64_t K = W[0]->K;
     rc = ensure_scratch2(c, (size_t)T * K * sizeof(float));
@@ -1543,13 +1566,14 @@ int spq4k_mul_mat_swiglu(spq4k_ctx* c, const spq4k_weights* Wg, const spq4k_weig
     }
     // unfused: [normalised rows], gate and up, then silu(gate) * up
     const int64_t K = Wg->K, M = Wg->M;
-    const size_t xb = norm_w ? (((size_t)T * K * sizeof(float) + 255) & ~(size_t)255) : 0;
+    const bool in_planes = norm_w && norm_in_planes(c, Wg, T);
+    const size_t xb = norm_w && !in_planes ? (((size_t)T * K * sizeof(float) + 255) & ~(size_t)255) : 0;
     const size_t gb = (((size_t)T * M * sizeof(float)) + 255) & ~(size_t)255;
     rc = ensure_scratch2(c, xb + 2 * gb);
     if (rc) return rc;
     const float* xin = x;
     hipError_t e;
-    if (norm_w) {
+    if (norm_w && !in_planes) {
         float* xn = reinterpret_cast<float*>(c->scratch2);
         e = launch_rms_norm(x, K, (int)T, (int)K, norm_w, eps, xn, c->stream);
         if (e != hipSuccess) return hip_fail(c, e, "rms_norm launch");
@@ -1558,7 +1582,8 @@ int spq4k_mul_mat_swiglu(spq4k_ctx* c, const spq4k_weights* Wg, const spq4k_weig
     float* G = reinterpret_cast<float*>(c->scratch2 + xb);
     float* U = reinterpret_cast<float*>(c->scratch2 + xb + gb);
     float* gu[2] = {G, U};
-    rc = mul_mat_n(c, 2, W, xin, gu, T);
+    const Norm nm = {norm_w, eps};
+    rc = mul_mat_n(c, 2, W, xin, gu, T, in_planes ? &nm : nullptr);
     if (rc) return rc;
     e = launch_swiglu(G, U, y, T * M, c->stream);
     if (e != hipSuccess) return hip_fail(c, e, "swiglu launch");

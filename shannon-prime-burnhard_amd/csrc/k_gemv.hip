@@ -503,25 +503,117 @@ __global__ __launch_bounds__(WAVES * 64) void gemv_decode_kernel(GemvParams p) {
     finish();
 }
 
-// RMS norm of T rows (one workgroup of 256 threads a row): the squares
+// RMS norm of T rows (one workgroup of 1024 threads a row): the squares
 // (fp32) summed in double by a fixed tree, mean = (float)(sum / K),
 // s = 1 / sqrtf(mean + eps), y = (x * s) * w (ggml-cpu/ops.cpp:3757-3779).
-__global__ __launch_bounds__(256) void rms_norm_kernel(const float* __restrict__ x, int64_t x_tstride, int K,
-                                                       const float* __restrict__ w, float eps,
-                                                       float* __restrict__ y) {
-    __shared__ double part[4];
-    const int t = blockIdx.x;
-    const float* xr = x + (int64_t)t * x_tstride;
-    double s = 0.0;
-    for (int k = threadIdx.x; k < K; k += 256) s += (double)(xr[k] * xr[k]);
+// Latency-bound: a row of 4096 is one 16-byte load a thread (VEC, all pointers
+// and the row stride 16-byte aligned). With 256 threads and scalar loads one
+// after another a launch took 13 us at any T up to 512.
+constexpr int NORM_THREADS = 1024;
+__device__ __forceinline__ float norm_scale(double s, int K, float eps, double* part, int nwave) {
     s = wave_sum_f64(s);
     if ((threadIdx.x & 63) == 0) part[threadIdx.x >> 6] = s;
     __syncthreads();
-    const double S = ((part[0] + part[1]) + part[2]) + part[3];
+    double S = part[0];
+    for (int i = 1; i < nwave; ++i) S += part[i];
     const float mean = (float)(S / (double)K);
-    const float scale = 1.0f / sqrtf(mean + eps);
+    return 1.0f / sqrtf(mean + eps);
+}
+template <bool VEC>
+__global__ __launch_bounds__(NORM_THREADS) void rms_norm_kernel(const float* __restrict__ x, int64_t x_tstride, int K,
+                                                                const float* __restrict__ w, float eps,
+                                                                float* __restrict__ y) {
+    __shared__ double part[NORM_THREADS / 64];
+    const int t = blockIdx.x;
+    const float* xr = x + (int64_t)t * x_tstride;
     float* yr = y + (int64_t)t * K;
-    for (int k = threadIdx.x; k < K; k += 256) yr[k] = xr[k] * scale * w[k];
+    double s = 0.0;
+    if constexpr (VEC) {
+        const float4* x4 = reinterpret_cast<const float4*>(xr);
+        for (int k = threadIdx.x; k < K / 4; k += NORM_THREADS) {
+            const float4 a = x4[k];
+            s += ((double)(a.x * a.x) + (double)(a.y * a.y)) + ((double)(a.z * a.z) + (double)(a.w * a.w));
+        }
+        const float scale = norm_scale(s, K, eps, part, NORM_THREADS / 64);
+        for (int k = threadIdx.x; k < K / 4; k += NORM_THREADS) {
+            const float4 a = x4[k], b = reinterpret_cast<const float4*>(w)[k];
+            reinterpret_cast<float4*>(yr)[k] =
+                make_float4(a.x * scale * b.x, a.y * scale * b.y, a.z * scale * b.z, a.w * scale * b.w);
+        }
+    } else {
+#pragma unroll 4
+        for (int k = threadIdx.x; k < K; k += NORM_THREADS) s += (double)(xr[k] * xr[k]);
+        const float scale = norm_scale(s, K, eps, part, NORM_THREADS / 64);
+        for (int k = threadIdx.x; k < K; k += NORM_THREADS) yr[k] = xr[k] * scale * w[k];
+    }
+}
+
+// The same norm with its Q8_K planes in one launch (the pre-norms of a batch):
+// a workgroup a row, 16 lanes a block, the row and the norm weights in
+// registers between the sum and the quantiser (P passes of NT / 16 blocks;
+// P = 0: a row too long for that is read twice). Launch-bound: the norm pass,
+// its rows' round trip and the planes pass were 13 + 4 us a call at T = 5 and
+// 15 + 6 us at T = 512 (4096 values), traced; this launch takes 4 and 8.
+template <int NT, int P>
+__global__ __launch_bounds__(NT) void rms_norm_planes_kernel(const float* __restrict__ x, int64_t x_tstride, int nb,
+                                                             const float* __restrict__ w, float eps,
+                                                             int8_t* __restrict__ qs, int16_t* __restrict__ bs,
+                                                             float* __restrict__ d, uint8_t* __restrict__ mn, int perm) {
+    __shared__ double part[NT / 64];
+    constexpr int B = NT / 16;            // blocks a pass
+    constexpr int NP = P > 0 ? P : 1;
+    const int64_t t = blockIdx.x;
+    const int e = threadIdx.x & 15, b0 = threadIdx.x >> 4;
+    const float* xr = x + t * x_tstride;
+    float v[NP][16], g[NP][16];
+    auto load = [&](const float* src, int b, float (&o)[16]) {   // rows past the end re-read the last block
+        const float4* p4 = reinterpret_cast<const float4*>(src + min(b, nb - 1) * QK + 16 * e);
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+            const float4 a = p4[i];
+            o[4 * i] = a.x; o[4 * i + 1] = a.y; o[4 * i + 2] = a.z; o[4 * i + 3] = a.w;
+        }
+    };
+    auto squares = [&](const float (&o)[16]) {
+        double a = 0.0, b = 0.0;
+#pragma unroll
+        for (int i = 0; i < 16; i += 2) {
+            a += (double)(o[i] * o[i]);
+            b += (double)(o[i + 1] * o[i + 1]);
+        }
+        return a + b;
+    };
+    double s = 0.0;
+    if constexpr (P > 0) {
+#pragma unroll
+        for (int p = 0; p < P; ++p) load(xr, b0 + p * B, v[p]);
+#pragma unroll
+        for (int p = 0; p < P; ++p) load(w, b0 + p * B, g[p]);
+#pragma unroll
+        for (int p = 0; p < P; ++p)
+            if (b0 + p * B < nb) s += squares(v[p]);
+    } else {
+        for (int b = b0; b < nb; b += B) {
+            load(xr, b, v[0]);
+            s += squares(v[0]);
+        }
+    }
+    const float scale = norm_scale(s, nb * QK, eps, part, NT / 64);
+    auto emit = [&](float (&o)[16], const float (&gw)[16], int b) {
+#pragma unroll
+        for (int i = 0; i < 16; ++i) o[i] = o[i] * scale * gw[i];
+        quantize_planes_item(o, e, t * nb + min(b, nb - 1), b < nb, qs, bs, d, mn, perm);
+    };
+    if constexpr (P > 0) {
+#pragma unroll
+        for (int p = 0; p < P; ++p) emit(v[p], g[p], b0 + p * B);
+    } else {
+        for (int b = b0; b < (nb + B - 1) / B * B; b += B) {   // whole passes: the quantiser exchanges lanes
+            load(xr, b, v[0]);
+            load(w, b, g[0]);
+            emit(v[0], g[0], b);
+        }
+    }
 }
 
 __global__ __launch_bounds__(256) void swiglu_kernel(const float* __restrict__ g, const float* __restrict__ u,
@@ -533,7 +625,25 @@ __global__ __launch_bounds__(256) void swiglu_kernel(const float* __restrict__ g
 hipError_t launch_rms_norm(const float* x, int64_t x_tstride, int T, int K, const float* w, float eps, float* y,
                            hipStream_t st) {
     if (T <= 0) return hipSuccess;
-    hipLaunchKernelGGL(rms_norm_kernel, dim3(T), dim3(256), 0, st, x, x_tstride, K, w, eps, y);
+    const bool vec = K % 4 == 0 && x_tstride % 4 == 0 && (((uintptr_t)x | (uintptr_t)w | (uintptr_t)y) & 15) == 0;
+    hipLaunchKernelGGL(vec ? rms_norm_kernel<true> : rms_norm_kernel<false>, dim3(T), dim3(NORM_THREADS), 0, st, x,
+                       x_tstride, K, w, eps, y);
+    return hipGetLastError();
+}
+
+hipError_t launch_rms_norm_planes(const float* x, int64_t x_tstride, int T, int nb, const float* w, float eps,
+                                  int8_t* qs, int16_t* bs, float* d, uint8_t* mn, bool perm, hipStream_t st) {
+    if (T <= 0) return hipSuccess;
+    // the fewest threads that hold the row in one pass; 128 blocks in two
+    const int lanes = nb * 16;
+    const auto go = [&](auto kernel, int nt) {
+        hipLaunchKernelGGL(kernel, dim3(T), dim3(nt), 0, st, x, x_tstride, nb, w, eps, qs, bs, d, mn, perm ? 1 : 0);
+    };
+    if (lanes <= 256) go(rms_norm_planes_kernel<256, 1>, 256);
+    else if (lanes <= 512) go(rms_norm_planes_kernel<512, 1>, 512);
+    else if (lanes <= 1024) go(rms_norm_planes_kernel<1024, 1>, 1024);
+    else if (lanes <= 2048) go(rms_norm_planes_kernel<1024, 2>, 1024);
+    else go(rms_norm_planes_kernel<1024, 0>, 1024);
     return hipGetLastError();
 }
 

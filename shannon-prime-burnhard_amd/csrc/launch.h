@@ -75,6 +75,10 @@ bool decode_fused_supported(int fmt, int nb, const DecodeCfg& c);
 // s_t = 1 / sqrt(mean(x[t]^2) + eps), one workgroup a row
 hipError_t launch_rms_norm(const float* x, int64_t x_tstride, int T, int K, const float* w, float eps, float* y,
                            hipStream_t st);
+// the same norm straight into Q8_K planes (rows of nb blocks, as launch_quantize_q8k_planes
+// writes them of the normalised rows); x rows and w 16-byte aligned
+hipError_t launch_rms_norm_planes(const float* x, int64_t x_tstride, int T, int nb, const float* w, float eps,
+                                  int8_t* qs, int16_t* bs, float* d, uint8_t* mn, bool perm, hipStream_t st);
 // y = silu(g) * u element-wise (ggml_silu then ggml_mul, ggml_vec_swiglu_f32)
 hipError_t launch_swiglu(const float* g, const float* u, float* y, int64_t n, hipStream_t st);
 hipError_t launch_subblock_sums(const uint8_t* W, int M, int nb, const float* X, int32_t* S, hipStream_t st);

@@ -87,6 +87,41 @@ def test_mul_mat_rms_norm(ctx, oracle, qtype, T):
         np.testing.assert_array_equal(a.to_host().view(np.uint32), b.to_host().view(np.uint32))
 
 
+@pytest.mark.parametrize("K,T", [(256, 2), (4096, 5), (4352, 3), (16384, 2), (16640, 3), (32768, 2), (33024, 3)])
+def test_norm_in_planes(ctx, oracle, K, T):
+    """The norm inside the planes pass at the row lengths where its launch
+    shape changes (one pass of 256 / 512 / 1024 threads, two, and the rows read
+    twice), matvec (T = 2, 3) and matrix-core (T = 5) batches: bit for bit the
+    norm pass and the matmul run one after the other."""
+    from spq4k.hip import DeviceArray
+    rng = np.random.default_rng(K + T)
+    M = 48
+    W = _enc(oracle, TYPE_Q4_K, M, K, rng)
+    X, w = _inputs(rng, T, K)
+    X[0, 0], X[T - 1, K - 1] = 1e30, -40.0
+    wd = ctx.upload(W, M, K)
+    xd, nd, yd, y2, xn = (DeviceArray.from_host(X), DeviceArray.from_host(w), DeviceArray((T, M)), DeviceArray((T, M)),
+                          DeviceArray((T, K)))
+    ctx.mul_mat_rms_norm_dev([wd], xd.ptr, nd.ptr, EPS, [yd.ptr], T)
+    ctx.rms_norm_dev(xd.ptr, nd.ptr, EPS, xn.ptr, K, T)
+    ctx.mul_mat_dev(wd, xn.ptr, y2.ptr, T)
+    ctx.synchronize()
+    np.testing.assert_array_equal(yd.to_host().view(np.uint32), y2.to_host().view(np.uint32))
+
+
+def test_rms_norm_misaligned_rows(ctx, oracle):
+    """Rows whose length or start is not a multiple of 16 bytes take the scalar form."""
+    from spq4k.hip import DeviceArray
+    rng = np.random.default_rng(5)
+    for K, off in ((1030, 0), (1028, 1)):
+        X, w = _inputs(rng, 3, K)
+        xd, wd, yd = DeviceArray((3 * K + 1,)), DeviceArray.from_host(w), DeviceArray((3, K))
+        xd.copy_from(np.concatenate([np.zeros(off, np.float32), X.ravel(), np.zeros(1 - off, np.float32)]))
+        ctx.rms_norm_dev(xd.ptr + 4 * off, wd.ptr, EPS, yd.ptr, K, 3)
+        ctx.synchronize()
+        np.testing.assert_array_equal(yd.to_host().view(np.uint32), oracle.rms_norm(X, w, EPS).view(np.uint32))
+
+
 @pytest.mark.parametrize("qtype", [TYPE_Q4_K, TYPE_Q5_K, TYPE_Q6_K, TYPE_Q8_0])
 @pytest.mark.parametrize("T,norm", [(1, True), (1, False), (4, True), (12, False)])
 def test_mul_mat_swiglu(ctx, oracle, qtype, T, norm):
