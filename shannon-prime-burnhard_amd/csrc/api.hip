@@ -207,6 +207,15 @@ struct Norm {
     float eps;
 };
 
+// What a batch's matmul does besides the product, where its path can: the norm
+// of its input, and (two matrices, gate and up) silu(gate) * up into glu in
+// the pass that finishes the outputs, reported by glu_done.
+struct Around {
+    const Norm* norm = nullptr;
+    float* glu = nullptr;
+    bool glu_done = false;
+};
+
 // extra: bytes of scratch wanted behind the planes (at q8_planes_bytes)
 int q8_planes(spq4k_ctx* c, const float* x, int64_t x_tstride, int T, int nb, Q8Planes* Q, bool perm = false,
               size_t extra = 0, const Norm* norm = nullptr) {
@@ -309,7 +318,7 @@ DecodeCfg plan_decode(const spq4k_ctx* c, int fmt, int nb_rows, int64_t rows, bo
 }
 
 int gemm_segments(spq4k_ctx* c, int n, const spq4k_weights* const* W, const float* X, float* const* Y, int64_t T,
-                  int mode, const Norm* norm = nullptr);
+                  int mode, Around* around = nullptr);
 
 // A fusion asked of gemv_launch: the decode kernel's RMS-norm prologue
 // (norm_w) and / or its gate-up SiLU epilogue (glu: W[0] gate, W[1] up, y[0]
@@ -474,9 +483,9 @@ int q80_dense(spq4k_ctx* c, int n, const spq4k_weights* const* W, const float* X
     return 0;
 }
 
-// norm (K-quant weights, T > 1): x is normalised as its planes are made.
+// around->norm (K-quant weights, T > 1): x is normalised as its planes are made.
 int gemv_launch(spq4k_ctx* c, int n, const spq4k_weights* const* W, const float* x, float* const* y, int64_t T,
-                const Fuse* fuse = nullptr, const Norm* norm = nullptr) {
+                const Fuse* fuse = nullptr, Around* around = nullptr) {
     if (n < 1 || n > GEMV_MAX_SEG) return set_err(c, -EINVAL, "gemv: n=%d matrices (1..4)", n);
     if (T < 1 || T > SPQ4K_GEMV_MAX_T) return set_err(c, -EINVAL, "gemv: T=%lld (1..8)", (long long)T);
     if (!x || !aligned(x, 16)) return set_err(c, -EINVAL, "gemv: x null or not 16-byte aligned");
@@ -561,7 +570,7 @@ int gemv_launch(spq4k_ctx* c, int n, const spq4k_weights* const* W, const float*
         !(p.fmt != WF_Q4K && c->gemm_mode == 1)) {
         // 4 <= T <= 8: the sdot4 kernel's integer work grows with T while the
         // matrix cores' 16-token tile costs the same from T = 1 to 16
-        return gemm_segments(c, n, W, x, y, T, c->gemm_mode == 1 ? 1 : 0, norm);
+        return gemm_segments(c, n, W, x, y, T, c->gemm_mode == 1 ? 1 : 0, around);
     }
     const int cb_max = LDS_BUDGET / ((int)T * 292);
     p.chunk_blocks = p.nb < cb_max ? p.nb : cb_max;
@@ -570,9 +579,9 @@ int gemv_launch(spq4k_ctx* c, int n, const spq4k_weights* const* W, const float*
     bool preq = (int64_t)p.nb * T > 48;
     if (c->preq_mode == 1) preq = true;
     if (c->preq_mode == 2) preq = false;
-    if (norm) preq = true;
+    if (around && around->norm) preq = true;
     if (preq) {
-        int rc = q8_planes(c, x, K, (int)T, p.nb, &p.Q, false, 0, norm);
+        int rc = q8_planes(c, x, K, (int)T, p.nb, &p.Q, false, 0, around ? around->norm : nullptr);
         if (rc) return rc;
     }
     hipError_t e = launch_gemv(p, (int)T, bpr, (int)tiles, c->stream);
@@ -1213,7 +1222,8 @@ namespace {
 // callers): plan, quantise X once into the context scratch (with the partial
 // plane of a K split behind it), launch.
 int gemm_segments(spq4k_ctx* c, int n, const spq4k_weights* const* W, const float* X, float* const* Y, int64_t T,
-                  int mode, const Norm* norm) {
+                  int mode, Around* around) {
+    const Norm* norm = around ? around->norm : nullptr;
     if (W[0]->fmt == WF_Q80) return q80_dense(c, n, W, X, Y, T);
     const int64_t K = W[0]->K;
     GemmParams p;
@@ -1239,7 +1249,7 @@ int gemm_segments(spq4k_ctx* c, int n, const spq4k_weights* const* W, const floa
     if (tiles16 * ((T + 15) / 16) > (1ll << 31) - 1 || rows > (1ll << 31) - 1)
         return set_err(c, -EINVAL, "gemm: grid too large");
     if (!fmt_has_mfma(p.fmt) || (p.fmt != WF_Q4K && mode == 1)) {   // sdot4 kernels over 8-token slices
-        if (T <= SPQ4K_GEMV_MAX_T) return gemv_launch(c, n, W, X, Y, T, nullptr, norm);
+        if (T <= SPQ4K_GEMV_MAX_T) return gemv_launch(c, n, W, X, Y, T, nullptr, around);
         return gemv_chunked(c, n, W, X, Y, T, norm);
     }
     hipError_t e;
@@ -1259,6 +1269,10 @@ int gemm_segments(spq4k_ctx* c, int n, const spq4k_weights* const* W, const floa
     int rc = q8_planes(c, X, K, (int)T, p.nb, &p.Q, g.perm, g.partial_bytes, norm);
     if (rc) return rc;
     p.P = g.ksplit > 1 ? reinterpret_cast<float*>(c->scratch + planes) : nullptr;
+    if (around && around->glu) {
+        p.glu = around->glu;
+        around->glu_done = true;
+    }
     e = launch_gemm(p, c->stream);
     if (e != hipSuccess) return hip_fail(c, e, "gemm launch");
     return 0;
@@ -1488,9 +1502,9 @@ namespace {
 
 // matmul of n matrices sharing X, any T (spq4k_mul_mat's dispatch)
 int mul_mat_n(spq4k_ctx* c, int n, const spq4k_weights* const* W, const float* X, float* const* Y, int64_t T,
-              const Norm* norm = nullptr) {
-    if (T <= SPQ4K_GEMV_MAX_T) return gemv_launch(c, n, W, X, Y, T, nullptr, norm);
-    return gemm_segments(c, n, W, X, Y, T, c->gemm_mode, norm);
+              Around* around = nullptr) {
+    if (T <= SPQ4K_GEMV_MAX_T) return gemv_launch(c, n, W, X, Y, T, nullptr, around);
+    return gemm_segments(c, n, W, X, Y, T, c->gemm_mode, around);
 }
 
 // Whether a batch's norm runs in the pass that makes the activation planes:
@@ -1535,7 +1549,9 @@ int spq4k_mul_mat_rms_norm(spq4k_ctx* c, int n, const spq4k_weights* const* W, c
     }
     if (norm_in_planes(c, W[0], T)) {
         const Norm nm = {norm_w, eps};
-        return mul_mat_n(c, n, W, x, y, T, &nm);
+        Around around;
+        around.norm = &nm;
+        return mul_mat_n(c, n, W, x, y, T, &around);
     }
     // unfused: the normalised rows, then the matmul on them
     const int64_t K = W[0]->K;
@@ -1583,8 +1599,11 @@ int spq4k_mul_mat_swiglu(spq4k_ctx* c, const spq4k_weights* Wg, const spq4k_weig
     float* U = reinterpret_cast<float*>(c->scratch2 + xb + gb);
     float* gu[2] = {G, U};
     const Norm nm = {norm_w, eps};
-    rc = mul_mat_n(c, 2, W, xin, gu, T, in_planes ? &nm : nullptr);
-    if (rc) return rc;
+    Around around;
+    around.norm = in_planes ? &nm : nullptr;
+    around.glu = y;
+    rc = mul_mat_n(c, 2, W, xin, gu, T, &around);
+    if (rc || around.glu_done) return rc;
     e = launch_swiglu(G, U, y, T * M, c->stream);
     if (e != hipSuccess) return hip_fail(c, e, "swiglu launch");
     return 0;

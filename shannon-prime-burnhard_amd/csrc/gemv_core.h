@@ -162,6 +162,9 @@ __device__ __forceinline__ void quantize_planes_items(const float* __restrict__ 
     quantize_planes_item(v, e, item, valid, qs, bs, d, mn, perm);
 }
 
+// silu(x) = x / (1 + e^-x) (ggml_silu_f32, ggml-cpu/vec.h:1064-1066)
+__device__ __forceinline__ float silu_f32(float x) { return x / (1.0f + expf(-x)); }
+
 // Two integer sub-block sums of one lane against one staged activation block.
 __device__ __forceinline__ void subblock_pair(const Nib& n, const int8_t* q8blk, int l4, int& S0, int& S1) {
     const int4* p = reinterpret_cast<const int4*>(q8blk + 64 * l4);

@@ -498,23 +498,38 @@ __global__ __launch_bounds__(NW * 64) void gemm_ring_kernel(GemmParams p) {
     }
 }
 
-// Y[t][r] of each segment = sum over the K ranges, in range order, of the
-// partial plane P[range][t][row_begin + r]: one element a thread, every
-// range's load issued before the sums.
+// Sum over the K ranges, in range order, of element i of the partial plane
+// (n elements a range): every range's load issued before the sums.
 constexpr int REDUCE_MAX_SPLIT = 32;
-__global__ __launch_bounds__(256) void gemm_reduce_kernel(GemmParams p) {
-    const int64_t n = (int64_t)p.T * p.rows;
-    const int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x;
-    if (i >= n) return;
-    const int ks = p.ksplit;
+__device__ __forceinline__ float reduce_ranges(const float* __restrict__ P, int64_t n, int64_t i, int ks) {
     float part[REDUCE_MAX_SPLIT];
 #pragma unroll
     for (int k = 0; k < REDUCE_MAX_SPLIT; ++k)
-        if (k < ks) part[k] = p.P[(int64_t)k * n + i];
+        if (k < ks) part[k] = P[(int64_t)k * n + i];
     float sum = part[0];
 #pragma unroll
     for (int k = 1; k < REDUCE_MAX_SPLIT; ++k)
         if (k < ks) sum += part[k];
+    return sum;
+}
+
+// Y[t][r] of each segment = the ranges' sum of P[range][t][row_begin + r]: one
+// element a thread. With p.glu (two segments of equal rows, gate and up) a
+// thread sums both rows of its element and stores silu(gate) * up there: the
+// element-wise pass and the round trip of both outputs go.
+__global__ __launch_bounds__(256) void gemm_reduce_kernel(GemmParams p) {
+    const int64_t n = (int64_t)p.T * p.rows;
+    const int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x;
+    if (p.glu) {
+        const int M = p.seg[0].M;
+        if (i >= n / 2) return;
+        const int64_t t = i / M, at = t * p.rows + (i - t * M);
+        const float g = reduce_ranges(p.P, n, at, p.ksplit), u = reduce_ranges(p.P, n, at + M, p.ksplit);
+        p.glu[i] = silu_f32(g) * u;
+        return;
+    }
+    if (i >= n) return;
+    const float sum = reduce_ranges(p.P, n, i, p.ksplit);
     const int t = (int)(i / p.rows);
     const int rg = (int)(i - (int64_t)t * p.rows);
     int sidx = 0;
@@ -877,8 +892,9 @@ hipError_t launch_gemm(const GemmParams& p0, hipStream_t st) {
     const int64_t grid = tiles * ((p.T + s.tok - 1) / s.tok) * p.ksplit;
     if (grid > INT32_MAX) return hipErrorInvalidValue;
     hipError_t e = s.launch(p, (int)grid, st);
-    if (e != hipSuccess || p.ksplit == 1) return e;
-    const int64_t n = (int64_t)p.T * p.rows;
+    if (e != hipSuccess) return e;
+    if (p.ksplit == 1) return p.glu ? launch_swiglu(p.seg[0].Y, p.seg[1].Y, p.glu, (int64_t)p.T * p.seg[0].M, st) : e;
+    const int64_t n = (int64_t)p.T * (p.glu ? p.rows / 2 : p.rows);
     hipLaunchKernelGGL(gemm_reduce_kernel, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, st, p);
     return hipGetLastError();
 }

@@ -107,9 +107,6 @@ __device__ __forceinline__ double wave_sum_f64(double v) {
     return v;
 }
 
-// silu(x) = x / (1 + e^-x) (ggml_silu_f32, ggml-cpu/vec.h:1064-1066)
-__device__ __forceinline__ float silu_f32(float x) { return x / (1.0f + expf(-x)); }
-
 // T = 1 decode kernel. One wave per output row: lane (bsub, l4) = (lane >> 2,
 // lane & 3) takes quarter l4 of blocks bsub, bsub + 16, ... of the row, so the
 // Q8_K data those quarters need is loaded into registers once and reused for

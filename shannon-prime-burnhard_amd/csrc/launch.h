@@ -192,6 +192,9 @@ struct GemmParams {
     int32_t kchunk;     // super-blocks per K range
     float* P;           // [ksplit][T][rows] partial plane when ksplit > 1
     int32_t fmt;        // WFmt of every segment (shapes are per format)
+    // two segments of equal M, gate and up: silu(gate) * up [T][M] goes here (their
+    // own outputs Y are then scratch that a K split leaves unwritten)
+    float* glu;
 };
 // Launch plan of the tiled / ring kernels for a GemmParams (T, nb, segments,
 // cfg): shape, K split and the scratch the partial plane needs.

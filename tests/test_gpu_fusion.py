@@ -109,6 +109,24 @@ def test_norm_in_planes(ctx, oracle, K, T):
     np.testing.assert_array_equal(yd.to_host().view(np.uint32), y2.to_host().view(np.uint32))
 
 
+@pytest.mark.parametrize("K", [1024, 4096])
+def test_swiglu_in_reduction(ctx, oracle, K):
+    """silu(gate) * up with one K range (its own pass) and with several (in
+    the pass that sums the ranges), ragged rows and tokens: bit for bit the
+    two matrices and spq4k_swiglu run one after the other."""
+    from spq4k.hip import DeviceArray
+    rng = np.random.default_rng(K)
+    M, T = 147, 19
+    g, u = (ctx.upload(_enc(oracle, TYPE_Q4_K, M, K, rng), M, K) for _ in range(2))
+    X, _ = _inputs(rng, T, K)
+    xd, yd, gd, ud, y2 = (DeviceArray.from_host(X),) + tuple(DeviceArray((T, M)) for _ in range(4))
+    ctx.mul_mat_swiglu_dev(g, u, xd.ptr, None, EPS, yd.ptr, T)
+    ctx.gemm_multi_dev([g, u], xd.ptr, [gd.ptr, ud.ptr], T)
+    ctx.swiglu_dev(gd.ptr, ud.ptr, y2.ptr, T * M)
+    ctx.synchronize()
+    np.testing.assert_array_equal(yd.to_host().view(np.uint32), y2.to_host().view(np.uint32))
+
+
 def test_rms_norm_misaligned_rows(ctx, oracle):
     """Rows whose length or start is not a multiple of 16 bytes take the scalar form."""
     from spq4k.hip import DeviceArray
