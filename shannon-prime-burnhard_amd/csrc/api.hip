@@ -132,12 +132,31 @@ size_t type_align(int type) { return type == SPQ4K_TYPE_Q4_K || type == SPQ4K_TY
 bool fmt_has_mfma(int fmt) { return fmt == WF_Q4K || fmt == WF_Q6K || fmt == WF_Q5K; }
 // formats of the expert-gathered ring kernel (moe_ring_kernel)
 bool fmt_has_moe_ring(int fmt) { return fmt == WF_Q4K || fmt == WF_Q6K || fmt == WF_Q5K; }
-// Waves of the expert ring kernel, measured on the 128-expert down bank at
-// T = 32 (us, 4 / 8 waves): Q6_K 54.9 / 59.9, Q5_K 45.0 / 48.0; Q4_K (the
-// MoE layer) 97.0 / 88.7 and Q8_0 70.2 / 67.6 keep 8.
-int moe_ring_waves(const spq4k_ctx* c, int fmt) {
-    if (c->moe_ring_waves) return c->moe_ring_waves;
-    return fmt == WF_Q6K || fmt == WF_Q5K ? 4 : 8;
+// Shape of the expert ring kernel by the pairs an active expert receives on
+// average: 16-pair tiles a workgroup takes at a time (ct) and waves (16 rows
+// each). An expert of more pairs than a workgroup takes is streamed again for
+// the rest; a wider tile holds fewer stages in LDS, so fewer bytes in flight.
+// Measured (us, the routed-expert block of 128 experts, top-8, 2048 -> 768,
+// ct = 1 with 8 waves / ct = 2 / ct = 4 with 4): Q4_K at 6 pairs 103 / 120 /
+// 153, 8 pairs 124 / 123 / 155, 12.5 pairs 158 / 133 / 163; 32 experts at 64
+// pairs 126 / 113 / 108; 60 experts of 3072 -> 1536 at 25 pairs 283 / 285 / 286
+// with 4 waves, and ct = 2 / 4 with 8 waves 248 / 238. Q6_K down bank in the
+// same block (8 waves for ct = 2): 8 pairs 145 / 150, 10 pairs 176 / 152,
+// 32 experts at 32 pairs 96 / 95 / 69. One pair tile, 4 / 8 waves (down bank,
+// T = 32): Q6_K 54.9 / 59.9, Q5_K 45.0 / 48.0, Q4_K (the MoE layer)
+// 97.0 / 88.7, Q8_0 70.2 / 67.6.
+struct MoeRingShape {
+    int ct, waves;
+};
+MoeRingShape moe_ring_shape(const spq4k_ctx* c, int fmt, int64_t mean_pairs, int nb) {
+    MoeRingShape s;
+    s.ct = fmt == WF_Q80 || mean_pairs <= 8 ? 1 : mean_pairs <= 20 ? 2 : 4;
+    if (s.ct == 1) s.waves = fmt == WF_Q6K || fmt == WF_Q5K ? 4 : 8;
+    else if (s.ct == 2) s.waves = fmt == WF_Q6K ? 8 : 4;
+    else s.waves = fmt == WF_Q4K && nb > 8 ? 8 : 4;
+    // a forced wave count (SPQ4K_MOE_RING_WAVES) takes the nearest instance
+    if (c->moe_ring_waves) s.waves = fmt == WF_Q5K && s.ct > 1 ? 4 : c->moe_ring_waves;
+    return s;
 }
 
 int use_device(spq4k_ctx* c) {
@@ -1442,7 +1461,7 @@ int q80_moe(spq4k_ctx* c, const spq4k_weights* const* banks, int nbank, const in
             mp.bank1 = banks[1]->data;
             mp.Y1 = Ys[1];
         }
-        const int nw = moe_ring_waves(c, WF_Q80);
+        const int nw = moe_ring_shape(c, WF_Q80, mean_pairs, mp.nb).waves;
         const int64_t ntiles = (M + 16 * nw - 1) / (16 * nw);
         int64_t rtw = ntiles * max_act * nbank / (2 * (int64_t)c->num_cus);
         if (rtw < 1) rtw = 1;
@@ -1792,7 +1811,9 @@ int moe_ring_run(spq4k_ctx* c, const spq4k_weights* const* banks, int nbank, con
     }
     // row tiles a workgroup streams: as many as still leave two workgroups
     // per CU over the experts (of every bank) that can be active
-    const int nw = moe_ring_waves(c, bank->fmt);
+    const MoeRingShape rs = moe_ring_shape(c, bank->fmt, (n_pairs + max_act - 1) / max_act, nb);
+    const int nw = rs.waves;
+    p.ring_ct = rs.ct;
     const int64_t ntiles = (M + 16 * nw - 1) / (16 * nw);
     int64_t rtw = ntiles * max_act * nbank / (2 * (int64_t)c->num_cus);
     if (rtw < 1) rtw = 1;

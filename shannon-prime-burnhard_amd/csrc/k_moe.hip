@@ -798,7 +798,7 @@ hipError_t launch_moe_gemv(const MoeParams& p, int tc, int bpr, int grid, hipStr
 //   moe_prep_kernel: workgroup 0 builds the routing tables (route_block), the
 //   others quantise the input rows into permuted Q8_K planes.
 //   moe_ring_kernel: workgroup (a, g) takes active expert a and its 128-row
-//   tiles g*ring_rt .. +ring_rt; the expert's pairs are gathered 16 at a time
+//   tiles g*ring_rt .. +ring_rt; the expert's pairs are gathered 16 CT at a time
 //   as the tokens of the LDS ring of gemm_ring_kernel (eight waves, one
 //   16-row tile each, direct global -> LDS loads S - 1 super-blocks ahead)
 //   and the row tiles follow each other in one stream, so the ring stays full
@@ -820,9 +820,9 @@ __global__ __launch_bounds__(256) void moe_prep_kernel(const int32_t* __restrict
 // F = 3: Q8_0 banks with K a multiple of 256 (17 slots: eight 34-byte
 // blocks; Q8_0 planes, the token's eight scales in its min-term slots;
 // ring_block_q80); as in gemm_ring_kernel.
-template <int S, int F = 0, int NW = 8>
+template <int S, int F = 0, int NW = 8, int CT = 1>
 __global__ __launch_bounds__(NW * 64) void moe_ring_kernel(MoeParams p) {
-    constexpr int ROWS = 16 * NW, TOK = 16;   // a wave's 16 rows of each row tile
+    constexpr int ROWS = 16 * NW, TOK = 16 * CT;   // a wave's 16 rows of each row tile
     constexpr int WSL = F == 1 ? 14 : F == 2 ? 11 : F == 3 ? 17 : 9;
     constexpr int BB = F == 1 ? Q6K_BYTES : F == 2 ? Q5K_BYTES : F == 3 ? Q80_RING_ROW : Q4K_BYTES;
     constexpr int ROWB = 16 * WSL;
@@ -906,7 +906,9 @@ __global__ __launch_bounds__(NW * 64) void moe_ring_kernel(MoeParams p) {
                     (const void*)a_, (__attribute__((address_space(3))) void*)(lds[buf] + (NW * i + wave) * 1024), 16, 0, 0);
             }
         };
-        v4f acc[1][1] = {{v4f{0, 0, 0, 0}}};
+        v4f acc[1][CT];
+#pragma unroll
+        for (int ct = 0; ct < CT; ++ct) acc[0][ct] = v4f{0, 0, 0, 0};
         // the previous token tile's readers are done with every buffer
         asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)\n\ts_barrier" ::: "memory");
 #pragma unroll
@@ -915,29 +917,30 @@ __global__ __launch_bounds__(NW * 64) void moe_ring_kernel(MoeParams p) {
             const int buf = sp % S;
             asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" ::"n"((S - 2) * NPW) : "memory");
             issue(min(sp + S - 1, len - 1), (sp + S - 1) % S);
-            if constexpr (F == 1)
-                ring_block_q6<1, 1>(lds[buf] + (wave * 16) * ROWB, lds[buf] + Q_OFF, lds[buf] + M_OFF, c16, q, acc);
-            else if constexpr (F == 2)
-                ring_block_q5<1, 1>(lds[buf] + (wave * 16) * ROWB, lds[buf] + Q_OFF, lds[buf] + M_OFF, c16, q, acc);
-            else if constexpr (F == 3)
-                ring_block_q80<1, 1>(lds[buf] + (wave * 16) * ROWB, lds[buf] + Q_OFF, lds[buf] + M_OFF, c16, q, acc);
-            else
-                ring_block<1, 1>(lds[buf] + (wave * 16) * Q4K_BYTES, lds[buf] + Q_OFF, lds[buf] + M_OFF, c16, q, acc);
+            const uint8_t* wl = lds[buf] + (wave * 16) * ROWB;
+            if constexpr (F == 1) ring_block_q6<1, CT>(wl, lds[buf] + Q_OFF, lds[buf] + M_OFF, c16, q, acc);
+            else if constexpr (F == 2) ring_block_q5<1, CT>(wl, lds[buf] + Q_OFF, lds[buf] + M_OFF, c16, q, acc);
+            else if constexpr (F == 3) ring_block_q80<1, CT>(wl, lds[buf] + Q_OFF, lds[buf] + M_OFF, c16, q, acc);
+            else ring_block<1, CT>(wl, lds[buf] + Q_OFF, lds[buf] + M_OFF, c16, q, acc);
             if (sp - (sp / nb) * nb == nb - 1) {
-                // row tile done: lane has rows 4q .. 4q+3 of the wave's 16, pair tile0 + c16
-                if (tile0 + c16 < pcnt) {
-                    const int pid = p.route.pairs[poff + tile0 + c16];
-                    const int rq = (rt0 + sp / nb) * ROWS + wave * 16 + 4 * q;
-                    float* y = Yb + (int64_t)pid * M + rq;
-                    if ((M & 3) == 0 && rq + 3 < M) {
-                        *reinterpret_cast<v4f*>(y) = acc[0][0];
-                    } else {
+                // row tile done: lane has rows 4q .. 4q+3 of the wave's 16, pairs tile0 + 16 ct + c16
+                const int rq = (rt0 + sp / nb) * ROWS + wave * 16 + 4 * q;
 #pragma unroll
-                        for (int i = 0; i < 4; ++i)
-                            if (rq + i < M) y[i] = acc[0][0][i];
+                for (int ct = 0; ct < CT; ++ct) {
+                    const int pi = tile0 + 16 * ct + c16;
+                    if (pi < pcnt) {
+                        const int pid = p.route.pairs[poff + pi];
+                        float* y = Yb + (int64_t)pid * M + rq;
+                        if ((M & 3) == 0 && rq + 3 < M) {
+                            *reinterpret_cast<v4f*>(y) = acc[0][ct];
+                        } else {
+#pragma unroll
+                            for (int i = 0; i < 4; ++i)
+                                if (rq + i < M) y[i] = acc[0][ct][i];
+                        }
                     }
+                    acc[0][ct] = v4f{0, 0, 0, 0};
                 }
-                acc[0][0] = v4f{0, 0, 0, 0};
             }
         }
         asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
@@ -965,21 +968,29 @@ hipError_t launch_moe_ring(const MoeParams& p, const int32_t* ids, int n_pairs, 
     hipError_t e = hipGetLastError();
     if (e != hipSuccess) return e;
     const int64_t grid = (int64_t)max_act * p.tiles_per_expert * (p.nbank > 1 ? 2 : 1);
-    if (nw == 4) {
-        if (p.fmt == WF_Q6K)
-            hipLaunchKernelGGL((moe_ring_kernel<3, 1, 4>), dim3((unsigned)grid), dim3(256), 0, st, p);
-        else if (p.fmt == WF_Q5K)
-            hipLaunchKernelGGL((moe_ring_kernel<3, 2, 4>), dim3((unsigned)grid), dim3(256), 0, st, p);
-        else
-            hipLaunchKernelGGL((moe_ring_kernel<3, 0, 4>), dim3((unsigned)grid), dim3(256), 0, st, p);
-    } else if (p.fmt == WF_Q6K) {
-        hipLaunchKernelGGL((moe_ring_kernel<3, 1, 8>), dim3((unsigned)grid), dim3(512), 0, st, p);
-    } else if (p.fmt == WF_Q5K) {
-        hipLaunchKernelGGL((moe_ring_kernel<3, 2, 8>), dim3((unsigned)grid), dim3(512), 0, st, p);
-    } else {
-        hipLaunchKernelGGL((moe_ring_kernel<3, 0, 8>), dim3((unsigned)grid), dim3(512), 0, st, p);
+    const auto go = [&](auto kernel) {
+        hipLaunchKernelGGL(kernel, dim3((unsigned)grid), dim3(nw * 64), 0, st, p);
+        return hipGetLastError();
+    };
+    switch (p.fmt * 100 + nw * 10 + p.ring_ct) {
+        case WF_Q4K * 100 + 41: return go(moe_ring_kernel<3, 0, 4, 1>);
+        case WF_Q4K * 100 + 42: return go(moe_ring_kernel<3, 0, 4, 2>);
+        case WF_Q4K * 100 + 44: return go(moe_ring_kernel<2, 0, 4, 4>);
+        case WF_Q4K * 100 + 81: return go(moe_ring_kernel<3, 0, 8, 1>);
+        case WF_Q4K * 100 + 82: return go(moe_ring_kernel<2, 0, 8, 2>);
+        case WF_Q4K * 100 + 84: return go(moe_ring_kernel<2, 0, 8, 4>);
+        case WF_Q6K * 100 + 41: return go(moe_ring_kernel<3, 1, 4, 1>);
+        case WF_Q6K * 100 + 42: return go(moe_ring_kernel<3, 1, 4, 2>);
+        case WF_Q6K * 100 + 44: return go(moe_ring_kernel<2, 1, 4, 4>);
+        case WF_Q6K * 100 + 81: return go(moe_ring_kernel<3, 1, 8, 1>);
+        case WF_Q6K * 100 + 82: return go(moe_ring_kernel<2, 1, 8, 2>);
+        case WF_Q6K * 100 + 84: return go(moe_ring_kernel<2, 1, 8, 4>);
+        case WF_Q5K * 100 + 41: return go(moe_ring_kernel<3, 2, 4, 1>);
+        case WF_Q5K * 100 + 42: return go(moe_ring_kernel<3, 2, 4, 2>);
+        case WF_Q5K * 100 + 44: return go(moe_ring_kernel<2, 2, 4, 4>);
+        case WF_Q5K * 100 + 81: return go(moe_ring_kernel<3, 2, 8, 1>);
     }
-    return hipGetLastError();
+    return hipErrorInvalidValue;
 }
 
 // The weighted sum over the routed experts that ends a MoE FFN block

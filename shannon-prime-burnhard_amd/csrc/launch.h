@@ -109,6 +109,7 @@ struct MoeParams {
     const uint8_t* bank1;
     float* Y1;
     int32_t nbank, max_act;
+    int32_t ring_ct;         // moe_ring_kernel: 16-pair tiles a workgroup takes at a time (1, 2 or 4)
 };
 
 hipError_t launch_moe_route(const int32_t* ids, int n_pairs, int E, const MoeRoute& r, hipStream_t st);

@@ -119,6 +119,33 @@ def test_moe_paths_agree(oracle, T, ne11, M, K):
         _check(got, exp, f"{env} T={T} ne11={ne11} M={M} K={K}")
 
 
+@pytest.mark.parametrize("qtype", [12, 13, 14])   # Q4_K, Q5_K, Q6_K
+@pytest.mark.parametrize("T,K", [(40, 768), (40, 2560), (150, 768), (150, 2560)])
+def test_moe_pair_tiles(oracle, qtype, T, K):
+    """Experts of about 13 and 50 pairs, which take two and four 16-pair tiles
+    of a workgroup at a time (uneven, some partly empty; ragged rows), short
+    and long rows: element-wise against the oracle, and bit for bit against a
+    forced wave count (the tiles hold the same sums)."""
+    from _envctx import context_with
+    E, k, M = 6, 2, 147
+    rng = np.random.default_rng(qtype + T + K)
+    W = oracle.quantize(qtype, (rng.standard_normal((E * M, K)) * 0.02).astype(np.float32))
+    X = rng.standard_normal((T, 1, K)).astype(np.float32)
+    ids = np.argsort(-(rng.standard_normal((T, E)) + np.linspace(0, 1.5, E)), axis=1)[:, :k].astype(np.int32)
+    outs = []
+    for env in ({}, {"SPQ4K_MOE_RING_WAVES": 4}, {"SPQ4K_MOE_RING_WAVES": 8}):
+        c = context_with(env)
+        try:
+            bank = c.upload(W, M, K, E, type=qtype)
+            outs.append(c.mul_mat_id(bank, X, ids))
+            bank.free()
+        finally:
+            c.close()
+    _check(outs[0], oracle.mul_mat_id_type(qtype, W, M, K, E, X, ids), f"type {qtype} T={T} K={K}")
+    for o in outs[1:]:
+        np.testing.assert_array_equal(outs[0].view(np.uint32), o.view(np.uint32))
+
+
 @pytest.mark.parametrize("mode", [0, 2, 3])
 def test_moe_device_ids_out_of_range_leave_outputs(oracle, mode):
     """Device-pointer entry point: an id outside [0, E) is not routed, so its
