@@ -32,6 +32,15 @@ using namespace spq4k;
 constexpr size_t KSPLIT_PARTIAL_BYTES = (size_t)8 << 20;
 static_assert(SPQ4K_NOALLOC_SCRATCH_BYTES - SPQ4K_NOALLOC_PLANES_MAX == KSPLIT_PARTIAL_BYTES,
               "the no-allocation scratch leaves a K split its whole budget");
+// Scratch a context starts with. A matmul whose planes fit it splits K only as
+// far as the partial plane fits beside them, so that its call never grows a
+// fresh context's scratch (which a call under capture may not do).
+constexpr size_t INITIAL_SCRATCH_BYTES = (size_t)16 << 20;
+constexpr size_t ksplit_budget(size_t planes) {
+    return planes >= INITIAL_SCRATCH_BYTES || INITIAL_SCRATCH_BYTES - planes >= KSPLIT_PARTIAL_BYTES
+               ? KSPLIT_PARTIAL_BYTES
+               : INITIAL_SCRATCH_BYTES - planes;
+}
 
 
 struct spq4k_ctx {
@@ -410,7 +419,7 @@ int q80_gemm(spq4k_ctx* c, int n, const spq4k_weights* const* W, const float* X,
     if ((rows + 15) / 16 * ((T + 15) / 16) > (1ll << 31) - 1 || rows > (1ll << 31) - 1)
         return set_err(c, -EINVAL, "gemm: grid too large");
     const size_t planes = q80_planes_bytes(T, nb);
-    const GemmPlan g = gemm_plan(p, c->num_cus, KSPLIT_PARTIAL_BYTES);
+    const GemmPlan g = gemm_plan(p, c->num_cus, ksplit_budget(planes));
     p.cfg = g.cfg;
     p.ksplit = g.ksplit;
     p.kchunk = g.kchunk;
@@ -790,7 +799,7 @@ int spq4k_init(int device, spq4k_ctx** out) {
     (void)noalloc_scratch_setup(device);
     // scratch for Q8_K activation planes: sized for prefill batches up front
     // so that steady-state calls (and graph capture) never allocate
-    if (ensure_scratch(c, (size_t)16 << 20) != 0 || ensure_scratch2(c, (size_t)4 << 20) != 0) {
+    if (ensure_scratch(c, INITIAL_SCRATCH_BYTES) != 0 || ensure_scratch2(c, (size_t)4 << 20) != 0) {
         if (c->scratch) (void)hipFree(c->scratch);
         if (c->scratch2) (void)hipFree(c->scratch2);
         (void)hipStreamDestroy(c->own_stream);
@@ -1281,7 +1290,7 @@ int gemm_segments(spq4k_ctx* c, int n, const spq4k_weights* const* W, const floa
         return 0;
     }
     const size_t planes = q8_planes_bytes((int)T, p.nb);
-    const GemmPlan g = gemm_plan(p, c->num_cus, KSPLIT_PARTIAL_BYTES);
+    const GemmPlan g = gemm_plan(p, c->num_cus, ksplit_budget(planes));
     p.cfg = g.cfg;
     p.ksplit = g.ksplit;
     p.kchunk = g.kchunk;

@@ -788,91 +788,75 @@ static int64_t row_tiles(const GemmParams& p, int rows) {
     return tiles;
 }
 
+// What a launch shape costs, measured on an MI355X (256 CUs, cold weights, one
+// K range, 8 and 24 super-blocks a row; us): `t1`, a super-block's step of a
+// launch with one workgroup a CU; `tn`, of one with `occ` workgroups a CU (as
+// many as its LDS leaves room for). Shapes that no size prefers are not listed.
+struct ShapeCost {
+    int cfg, occ;
+    float t1, tn;
+};
+static const ShapeCost kCostQ4K[] = {{8, 3, 0.60f, 1.45f}, {6, 2, 0.90f, 1.86f}, {7, 1, 1.15f, 1.15f},
+                                     {1, 1, 1.70f, 1.70f}, {32, 2, 1.76f, 3.14f}, {11, 1, 3.13f, 3.13f}};
+static const ShapeCost kCostQ6K[] = {{29, 2, 0.92f, 1.57f}, {18, 1, 1.65f, 1.65f}, {16, 1, 1.79f, 1.79f},
+                                     {14, 1, 2.20f, 2.20f}, {17, 1, 4.66f, 4.66f}};
+static const ShapeCost kCostQ5K[] = {{30, 2, 0.80f, 1.28f}, {20, 1, 1.21f, 1.21f}, {23, 1, 1.34f, 1.34f},
+                                     {21, 1, 1.60f, 1.60f}, {19, 1, 2.19f, 2.19f}};
+static const ShapeCost kCostQ80[] = {{31, 2, 1.77f, 2.04f}, {28, 2, 2.84f, 3.61f}, {27, 1, 3.83f, 3.83f},
+                                     {26, 1, 4.98f, 4.98f}};
+
+// The launch shape and K split of least estimated time. A launch runs in
+// rounds of occ workgroups a CU; a round costs its fill and drain (4 us: the
+// 512-tile runs of the sweep above against the 256-tile ones) and a step a
+// super-block, the last round less when it leaves CUs (or their second place)
+// empty; a K split adds the reduction pass (3 us and its bytes at 3.5 TB/s). So
+// a grid a little over a whole number of rounds takes fewer ranges or another
+// tile instead: 4096 x 12288 Q6_K at T = 100 ran 320 workgroups, one a CU, in
+// two rounds of ten super-blocks; four ranges make one of twelve.
 GemmPlan gemm_plan(const GemmParams& p, int num_cus, size_t max_partial_bytes) {
+    const ShapeCost* cost = p.fmt == WF_Q6K ? kCostQ6K : p.fmt == WF_Q5K ? kCostQ5K : p.fmt == WF_Q80 ? kCostQ80 : kCostQ4K;
+    const int ncost = (int)(p.fmt == WF_Q6K   ? sizeof kCostQ6K
+                            : p.fmt == WF_Q5K ? sizeof kCostQ5K
+                            : p.fmt == WF_Q80 ? sizeof kCostQ80 : sizeof kCostQ4K) / (int)sizeof(ShapeCost);
+    const bool forced = p.cfg >= 0 && p.cfg < N_TILED && kTiled[p.cfg].fmt == p.fmt;   // not a shape of another format
+    const size_t per_split = (size_t)p.T * p.rows * sizeof(float);
+    int most = max_partial_bytes / per_split < REDUCE_MAX_SPLIT ? (int)(max_partial_bytes / per_split) : REDUCE_MAX_SPLIT;
+    if (most < 1) most = 1;
+
     GemmPlan g;
-    int cfg = p.cfg;
-    if (cfg >= 0 && cfg < N_TILED && kTiled[cfg].fmt != p.fmt) cfg = -1;   // a shape of the other format
-    // T <= 32 (Q8_0: T <= 16, or <= 32 on 4096 rows or fewer): 64 x 16 tiles
-    // of 4 waves, measured (us, against the 128-row shapes) at T = 16 on
-    // 24576 x 4096 / 4096 x 12288 / 1024 x 4096: Q6_K 34.1 / 22.3 / 13.1
-    // against 47.9 / 28.4 / 16.5, Q5_K 29.7 / 20.3 / 12.2 against
-    // 36.6 / 23.0 / 14.0, Q8_0 44.8 / 26.5 / 15.5 against 49.9 / 28.7 / 19.5;
-    // at T = 32 Q6_K 47.4 against 52.5 and Q5_K 37.9 against 46.2 on 24576
-    // rows, Q8_0 66.7 against 62.3 there
-    if ((cfg < 0 || cfg >= N_TILED) && p.fmt == WF_Q6K) {
-        cfg = p.T <= 32 ? 29 : 14;
-    } else if ((cfg < 0 || cfg >= N_TILED) && p.fmt == WF_Q5K) {
-        cfg = p.T <= 32 ? 30 : 19;
-    } else if ((cfg < 0 || cfg >= N_TILED) && p.fmt == WF_Q80) {
-        // above 32 tokens: 128 x 64 tiles, 2 stages (4096 x 12288 at T = 512:
-        // 227 us); 17..32 tokens on more than 4096 rows: 128 x 16, 2 stages
-        cfg = (p.T <= 16 || (p.T <= 32 && p.rows <= 4096)) ? 31 : (p.T <= 32 ? 28 : 26);
-    } else if (cfg < 0 || cfg >= N_TILED) {
-        // tall (12288 rows or more) or long-K (48 super-blocks or more)
-        const bool big = p.rows >= 12288 || p.nb >= 48;
-        // measured on the 8B shapes (us, the choice against the next best):
-        //   T = 16: 64 x 16 tiles, 4 waves: 24576 x 4096 24.5 / 28.3,
-        //           4096 x 12288 17.4 / 18.7, 4096 x 4096 12.5 / 13.4
-        //           (6144 x 4096 14.7 / 14.3);
-        //   T = 32: the same on big matrices (24576 rows 29.2 / 38.8,
-        //           4096 x 12288 21.4 / 23.6), 128 x 32 otherwise;
-        //   32 < T < 128: 32x32 tiles on big matrices (24576 rows at T = 64
-        //           41.4 / 48.2, 4096 x 12288 26.2 / 30.8), 128 x 32 on 4096
-        //           rows (16.8 / 19.2), else 128 x 64
-        if (p.T <= 16) {
-            cfg = 8;
-        } else if (p.T <= 32) {
-            cfg = big ? 8 : 7;
-        } else if (p.T < 128 && big) {
-            cfg = 11;
-        } else if (p.T < 128 && p.rows <= 4096) {
-            cfg = 7;
-        } else {
-            // the largest tile that gives every CU a workgroup without a K
-            // split, else 128 x 64 with one. Measured on MI355X at T = 512:
-            // 256 x 64 on 32x32 MFMA tiles for 24576 rows (140 us against 155
-            // on 16x16 tiles), 128 x 64 on 16x16 tiles for 4096 rows.
-            // From T = 128 the 32x32 tiles also win on matrices of 6144 rows
-            // or more (24 tiles of 256), measured at T = 128 / 512:
-            //   6144 x 4096: 29.1 / 52.1 us against 32.1 / 64.0;
-            //   24576 x 4096 at T = 128: 54.0 against 62.8.
-            // They lose at 4096 rows: 4096 x 4096 at T = 512 is 50.0 against
-            // 37.1, and 4096 x 12288 is 129 against 91.
-            cfg = 1;
-            const int64_t rt = row_tiles(p, 256);
-            const int64_t g0 = rt * ((p.T + 63) / 64);
-            if (g0 >= num_cus || (p.T >= 128 && rt >= 24)) cfg = 11;
-            // From T = 256 on 12288 rows or more: the same 32x32 tiles in
-            // 4-wave workgroups of 128 rows, two a CU, whose barriers do not
-            // hold all eight waves of a CU in step (24576 x 4096 at T = 512,
-            // cold weights: 164-165 against 169 us, in one run of both; 6144
-            // rows: 54.3 against 52.2; T = 128 on 24576 rows: 55.0 against
-            // 53.9)
-            if (cfg == 11 && p.T >= 256 && p.rows >= 12288) cfg = 32;
+    g.cfg = -1;
+    float best = 0.0f;
+    for (int k = 0; k < (forced ? 1 : ncost); ++k) {
+        ShapeCost c = cost[k];
+        if (forced) {   // its cost if it is listed, else any: only the split is chosen
+            c = {p.cfg, 1, 1.0f, 1.0f};
+            for (int m = 0; m < ncost; ++m)
+                if (cost[m].cfg == p.cfg) c = cost[m];
+        }
+        const TiledShape& s = kTiled[c.cfg];
+        const int64_t tiles = row_tiles(p, s.rows) * ((p.T + s.tok - 1) / s.tok);
+        const int64_t place = (int64_t)num_cus * c.occ;
+        for (int want = 1; want <= (s.ring ? most : 1) && want <= p.nb; ++want) {
+            const int kchunk = (p.nb + want - 1) / want, ks = (p.nb + kchunk - 1) / kchunk;
+            if (ks != want) continue;   // the same ranges as a smaller count
+            const int64_t wgs = tiles * ks, full = wgs / place, rem = wgs - full * place;
+            float step = full * c.tn;
+            if (rem > 0) {   // the fullest CU of the last round sets its pace
+                const int64_t on = (rem + num_cus - 1) / num_cus;
+                step += on == 1 ? c.t1 : c.t1 + (c.tn - c.t1) * (float)(on - 1) / (float)(c.occ - 1);
+            }
+            float us = 4.0f * (float)(full + (rem > 0)) + step * (float)kchunk;
+            if (ks > 1) us += 3.0f + (float)(ks + 1) * (float)per_split / 3.5e6f;
+            if (g.cfg < 0 || us < best) {
+                best = us;
+                g.cfg = c.cfg;
+                g.ksplit = ks;
+                g.kchunk = ks > 1 ? kchunk : p.nb;
+            }
         }
     }
-    const TiledShape& s = kTiled[cfg];
-    g.cfg = cfg;
-    g.perm = s.ring;
-    g.ksplit = 1;
-    g.kchunk = p.nb;
-    g.partial_bytes = 0;
-    if (s.ring) {
-        // split K until two workgroups per CU, keeping >= 4 super-blocks a range
-        const int64_t grid0 = row_tiles(p, s.rows) * ((p.T + s.tok - 1) / s.tok);
-        int64_t want = (2 * (int64_t)num_cus + grid0 - 1) / grid0;
-        int64_t most = p.nb / 4 > 1 ? p.nb / 4 : 1;
-        if (most > REDUCE_MAX_SPLIT) most = REDUCE_MAX_SPLIT;
-        if (want > most) want = most;
-        const size_t per_split = (size_t)p.T * p.rows * sizeof(float);
-        while (want > 1 && (size_t)want * per_split > max_partial_bytes) --want;
-        if (want > 1) {
-            g.kchunk = (int)((p.nb + want - 1) / want);
-            g.ksplit = (p.nb + g.kchunk - 1) / g.kchunk;
-            g.partial_bytes = g.ksplit > 1 ? (size_t)g.ksplit * per_split : 0;
-            if (g.ksplit == 1) g.kchunk = p.nb;
-        }
-    }
+    g.perm = kTiled[g.cfg].ring;
+    g.partial_bytes = g.ksplit > 1 ? (size_t)g.ksplit * per_split : 0;
     return g;
 }
 

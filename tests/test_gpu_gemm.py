@@ -208,3 +208,29 @@ def test_gemm_k_split_fixup(ctx, oracle, M, K, T, qtype):
     del g
     for a in (Wd, W2d, xd, yd):
         a.free()
+
+
+@pytest.mark.parametrize("qtype", [8, 12, 13, 14])   # Q8_0, Q4_K, Q5_K, Q6_K
+@pytest.mark.parametrize("M,nb,T", [(70, 5, 9), (1100, 7, 40), (520, 33, 100), (300, 11, 260), (4100, 3, 17)])
+def test_gemm_plan_ranges(ctx, oracle, M, nb, T, qtype):
+    """Shapes whose split leaves ranges of one super-block, a shorter last
+    range, or many ranges of few tiles (ragged rows and tokens): against the
+    oracle, and the no-allocation call (the same plan) bit for bit."""
+    from spq4k.hip import DeviceArray
+    K = 256 * nb
+    rng = np.random.default_rng(M + K + T + qtype)
+    Wf = (rng.standard_normal((M, K)) * 0.02).astype(np.float32)
+    X = rng.standard_normal((T, K)).astype(np.float32)
+    W = oracle.quantize_q8_0(Wf, ref_encoder=True) if qtype == 8 else oracle.quantize(qtype, Wf)
+    Wd = ctx.upload(W, M, K, type=qtype)
+    xd, yd, y2 = DeviceArray.from_host(X), DeviceArray((T, M)), DeviceArray((T, M))
+    ctx.mul_mat_dev(Wd, xd.ptr, yd.ptr, T)
+    assert ctx.lib.spq4k_mul_mat_noalloc(ctx.handle, Wd.handle, xd.ptr, y2.ptr, T) == 0
+    ctx.synchronize()
+    got = yd.to_host()
+    if qtype == 8:
+        _check(got, oracle.mul_mat_q8_0(W, M, K, X), f"Q8_0 M={M} K={K} T={T}")
+    else:
+        _check(got, oracle.mul_mat_type(qtype, W, M, K, X), f"type {qtype} M={M} K={K} T={T}",
+               oracle.mul_mat_dq_f64(qtype, W, M, K, X))
+    assert np.array_equal(got.view(np.uint32), y2.to_host().view(np.uint32))
