@@ -802,8 +802,8 @@ static const ShapeCost kCostQ6K[] = {{29, 2, 0.92f, 1.57f}, {18, 1, 1.65f, 1.65f
                                      {14, 1, 2.20f, 2.20f}, {17, 1, 4.66f, 4.66f}};
 static const ShapeCost kCostQ5K[] = {{30, 2, 0.80f, 1.28f}, {20, 1, 1.21f, 1.21f}, {23, 1, 1.34f, 1.34f},
                                      {21, 1, 1.60f, 1.60f}, {19, 1, 2.19f, 2.19f}};
-static const ShapeCost kCostQ80[] = {{31, 2, 1.77f, 2.04f}, {28, 2, 2.84f, 3.61f}, {27, 1, 3.83f, 3.83f},
-                                     {26, 1, 4.98f, 4.98f}};
+static const ShapeCost kCostQ80[] = {{31, 2, 1.40f, 1.74f}, {28, 2, 2.21f, 3.24f}, {27, 1, 3.37f, 3.37f},
+                                     {26, 1, 4.23f, 4.23f}};
 
 // The launch shape and K split of least estimated time. A launch runs in
 // rounds of occ workgroups a CU; a round costs its fill and drain (4 us: the
