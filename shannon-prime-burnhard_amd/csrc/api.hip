@@ -1281,7 +1281,7 @@ int gemm_segments(spq4k_ctx* c, int n, const spq4k_weights* const* W, const floa
         return gemv_chunked(c, n, W, X, Y, T, norm);
     }
     hipError_t e;
-    if (gemm_use_skinny((int)T, mode)) {
+    if (gemm_use_skinny(p, tiles16)) {
         int rc = q8_planes(c, X, K, (int)T, p.nb, &p.Q, false, 0, norm);
         if (rc) return rc;
         p.total_tiles = (int32_t)tiles16;

@@ -720,7 +720,20 @@ hipError_t launch_gemm_skinny(const GemmParams& p, hipStream_t st) {
     return longk ? launch_skinny<4, 16, 1>(p, st) : launch_skinny<4, 8, 1>(p, st);
 }
 
-bool gemm_use_skinny(int T, int mode) { return mode == 1; }
+// The skinny form takes what mode 1 forces, and small Q4_K matrices of at most
+// 16 tokens: its waves' sums meet in LDS, so no reduction launch follows, but
+// every 16 rows read all the activations and its waves wait for their loads
+// once a chunk. Measured (us, at T = 4 / 8 / 16, against the ring and its
+// reduction): 4096 x 2048 6.8 / 7.1 / 7.8 against 9.9 / 10.2 / 10.6,
+// 8192 x 2048 8.6 / 9.2 against 10.0 / 10.1, 4096 x 4096 9.0 / 9.7 / 10.5
+// against 11.3 / 11.4 / 11.9; not 1024 x 4096 (8.6 / 9.3 / 10.3 against
+// 9.4 / 9.3 / 9.7), 6144 x 4096 (12.8 / 14.2 / 16.5 against 13.2 / 13.7 / 14.7)
+// or 4096 x 8192 (12.8 / 14.2 against 13.7 / 14.1).
+bool gemm_use_skinny(const GemmParams& p, int64_t tiles16) {
+    if (p.mode == 1) return true;
+    if (p.mode != 0 || p.cfg >= 0 || p.fmt != WF_Q4K || p.T > 16) return false;
+    return p.nb <= 8 ? tiles16 <= 512 : p.nb <= 16 && tiles16 >= 128 && tiles16 <= 256;
+}
 
 // Tiled-kernel launch shapes, indexed by GemmParams::cfg (-1: chosen here).
 struct TiledShape {

@@ -205,7 +205,8 @@ struct GemmPlan {
     bool perm;                 // reads the permuted Q8_K values
     size_t partial_bytes;      // ksplit * T * rows * 4 when ksplit > 1
 };
-bool gemm_use_skinny(int T, int mode);
+// whether the matmul takes the skinny kernel (16-row tiles: tiles16 of them over all segments)
+bool gemm_use_skinny(const GemmParams& p, int64_t tiles16);
 int gemm_tiled_shapes();
 GemmPlan gemm_plan(const GemmParams& p, int num_cus, size_t max_partial_bytes);
 // p.cfg / p.ksplit / p.kchunk / p.P as planned; launches the reduction too

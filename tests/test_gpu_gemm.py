@@ -211,11 +211,12 @@ def test_gemm_k_split_fixup(ctx, oracle, M, K, T, qtype):
 
 
 @pytest.mark.parametrize("qtype", [8, 12, 13, 14])   # Q8_0, Q4_K, Q5_K, Q6_K
-@pytest.mark.parametrize("M,nb,T", [(70, 5, 9), (1100, 7, 40), (520, 33, 100), (300, 11, 260), (4100, 3, 17)])
+@pytest.mark.parametrize("M,nb,T", [(70, 5, 9), (1100, 7, 40), (520, 33, 100), (300, 11, 260), (4100, 3, 17),
+                                    (2060, 16, 5), (2100, 8, 16), (4111, 13, 16), (37, 1, 4)])
 def test_gemm_plan_ranges(ctx, oracle, M, nb, T, qtype):
     """Shapes whose split leaves ranges of one super-block, a shorter last
-    range, or many ranges of few tiles (ragged rows and tokens): against the
-    oracle, and the no-allocation call (the same plan) bit for bit."""
+    range, or many ranges of few tiles (ragged rows and tokens), and the
+    matrices small enough for the skinny kernel: against the oracle, and the no-allocation call (the same plan) bit for bit."""
     from spq4k.hip import DeviceArray
     K = 256 * nb
     rng = np.random.default_rng(M + K + T + qtype)
