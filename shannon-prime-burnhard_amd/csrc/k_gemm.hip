@@ -790,6 +790,19 @@ static const TiledShape kTiled[] = {
     {64, 16, true, launch_ring_<1, 1, 4, 3, 16, 2>, WF_Q5K},    // 30
     {64, 16, true, launch_ring_<1, 1, 4, 3, 16, 3>, WF_Q80},    // 31
     {128, 64, true, launch_ring_<1, 2, 4, 2, 32>},   // 32: ring 32x32, 4 waves, 2 stages (two workgroups a CU)
+    // 64-row tiles, 4 waves, 2 stages: two to four workgroups a CU, so that one's
+    // barriers do not hold the others' waves in step and a grid fills its last
+    // round better. A step of two 64 x 64 tiles a CU against one of 128 x 64 (us):
+    // Q8_0 3.54 / 4.23, Q4_K 1.76 / 1.70, Q6_K 2.27 / 2.20, Q5_K 2.33 / 2.19;
+    // 13824 x 5120 Q5_K at T = 150 runs 66.5 us against 86.7 with 128 x 64.
+    {64, 64, true, launch_ring_<1, 4, 4, 2>},                   // 33
+    {64, 64, true, launch_ring_<1, 4, 4, 2, 16, 1>, WF_Q6K},    // 34
+    {64, 64, true, launch_ring_<1, 4, 4, 2, 16, 2>, WF_Q5K},    // 35
+    {64, 64, true, launch_ring_<1, 4, 4, 2, 16, 3>, WF_Q80},    // 36
+    {64, 32, true, launch_ring_<1, 2, 4, 2>},                   // 37
+    {64, 32, true, launch_ring_<1, 2, 4, 2, 16, 1>, WF_Q6K},    // 38
+    {64, 32, true, launch_ring_<1, 2, 4, 2, 16, 2>, WF_Q5K},    // 39
+    {64, 32, true, launch_ring_<1, 2, 4, 2, 16, 3>, WF_Q80},    // 40
 };
 constexpr int N_TILED = (int)(sizeof(kTiled) / sizeof(kTiled[0]));
 
@@ -810,13 +823,16 @@ struct ShapeCost {
     float t1, tn;
 };
 static const ShapeCost kCostQ4K[] = {{8, 3, 0.60f, 1.45f}, {6, 2, 0.90f, 1.86f}, {7, 1, 1.15f, 1.15f},
-                                     {1, 1, 1.70f, 1.70f}, {32, 2, 1.76f, 3.14f}, {11, 1, 3.13f, 3.13f}};
+                                     {1, 1, 1.70f, 1.70f}, {32, 2, 1.76f, 3.14f}, {11, 1, 3.13f, 3.13f},
+                                     {37, 4, 0.80f, 2.54f}, {33, 2, 1.08f, 1.76f}};
 static const ShapeCost kCostQ6K[] = {{29, 2, 0.92f, 1.57f}, {18, 1, 1.65f, 1.65f}, {16, 1, 1.79f, 1.79f},
-                                     {14, 1, 2.20f, 2.20f}, {17, 1, 4.66f, 4.66f}};
+                                     {14, 1, 2.20f, 2.20f}, {17, 1, 4.66f, 4.66f}, {38, 2, 1.15f, 1.92f},
+                                     {34, 2, 1.57f, 2.27f}};
 static const ShapeCost kCostQ5K[] = {{30, 2, 0.80f, 1.28f}, {20, 1, 1.21f, 1.21f}, {23, 1, 1.34f, 1.34f},
-                                     {21, 1, 1.60f, 1.60f}, {19, 1, 2.19f, 2.19f}};
+                                     {21, 1, 1.60f, 1.60f}, {19, 1, 2.19f, 2.19f}, {39, 3, 0.94f, 2.25f},
+                                     {35, 2, 1.37f, 2.33f}};
 static const ShapeCost kCostQ80[] = {{31, 2, 1.40f, 1.74f}, {28, 2, 2.21f, 3.24f}, {27, 1, 3.37f, 3.37f},
-                                     {26, 1, 4.23f, 4.23f}};
+                                     {26, 1, 4.23f, 4.23f}, {40, 2, 1.83f, 2.01f}, {36, 2, 3.31f, 3.54f}};
 
 // The launch shape and K split of least estimated time. A launch runs in
 // rounds of occ workgroups a CU; a round costs its fill and drain (4 us: the

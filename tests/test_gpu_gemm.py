@@ -235,3 +235,24 @@ def test_gemm_plan_ranges(ctx, oracle, M, nb, T, qtype):
         _check(got, oracle.mul_mat_type(qtype, W, M, K, X), f"type {qtype} M={M} K={K} T={T}",
                oracle.mul_mat_dq_f64(qtype, W, M, K, X))
     assert np.array_equal(got.view(np.uint32), y2.to_host().view(np.uint32))
+
+
+@pytest.mark.parametrize("cfg", list(range(33, 41)))
+def test_gemm_two_stage_shapes(oracle, cfg):
+    """The 64-row two-stage launch shapes of each format (SPQ4K_GEMM_CFG) with
+    ragged rows, tokens and ranges, against the oracle."""
+    from _envctx import context_with
+    qtype = (12, 14, 13, 8)[(cfg - 33) % 4]
+    c = context_with({"SPQ4K_GEMM_CFG": cfg})
+    try:
+        rng = np.random.default_rng(cfg)
+        for M, K, T in ((130, 1280, 33), (67, 256, 65), (64, 4096, 9)):
+            Wf = (rng.standard_normal((M, K)) * 0.02).astype(np.float32)
+            X = rng.standard_normal((T, K)).astype(np.float32)
+            W = oracle.quantize_q8_0(Wf, ref_encoder=True) if qtype == 8 else oracle.quantize(qtype, Wf)
+            got = c.mul_mat(c.upload(W, M, K, type=qtype), X)
+            exp = oracle.mul_mat_q8_0(W, M, K, X) if qtype == 8 else oracle.mul_mat_type(qtype, W, M, K, X)
+            exact = None if qtype == 8 else oracle.mul_mat_dq_f64(qtype, W, M, K, X)
+            _check(got, exp, f"cfg={cfg} M={M} K={K} T={T}", exact)
+    finally:
+        c.close()
