@@ -342,7 +342,9 @@ int spq4k_moe_ffn_host(spq4k_ctx *ctx, const spq4k_weights *gate, const spq4k_we
  *                          matrices sharing the input (the attention and FFN
  *                          pre-norms, forward.cpp:1693-1696): at T = 1 one
  *                          launch, the norm in the matvec's prologue;
- *                          otherwise the norm pass, then spq4k_mul_mat's path.
+ *                          otherwise spq4k_mul_mat's path on the normalised
+ *                          rows (K-quant weights: the norm in the pass that
+ *                          quantises them).
  * spq4k_mul_mat_swiglu   : y = silu(Wg . xb) * (Wu . xb), xb = x, or
  *                          rms_norm(x) * norm_w when norm_w is not NULL (the
  *                          dense SwiGLU front half, forward.cpp:1703-1706;
