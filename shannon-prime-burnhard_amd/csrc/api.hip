@@ -153,7 +153,7 @@ bool fmt_has_moe_ring(int fmt) { return fmt == WF_Q4K || fmt == WF_Q6K || fmt ==
 // same block (8 waves for ct = 2): 8 pairs 145 / 150, 10 pairs 176 / 152,
 // 32 experts at 32 pairs 96 / 95 / 69. One pair tile, 4 / 8 waves (down bank,
 // T = 32): Q6_K 54.9 / 59.9, Q5_K 45.0 / 48.0, Q4_K (the MoE layer)
-// 97.0 / 88.7, Q8_0 70.2 / 67.6.
+// 97.0 / 88.7, Q8_0 64.2 / 57.4.
 struct MoeRingShape {
     int ct, waves;
 };
