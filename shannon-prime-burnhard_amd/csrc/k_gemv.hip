@@ -500,13 +500,12 @@ __global__ __launch_bounds__(WAVES * 64) void gemv_decode_kernel(GemvParams p) {
     finish();
 }
 
-// RMS norm of T rows (one workgroup of 1024 threads a row): the squares
-// (fp32) summed in double by a fixed tree, mean = (float)(sum / K),
+// RMS norm of rows, one workgroup of NT threads a row: the squares (fp32)
+// summed in double by a fixed tree, mean = (float)(sum / K),
 // s = 1 / sqrtf(mean + eps), y = (x * s) * w (ggml-cpu/ops.cpp:3757-3779).
 // Latency-bound: a row of 4096 is one 16-byte load a thread (VEC, all pointers
 // and the row stride 16-byte aligned). With 256 threads and scalar loads one
 // after another a launch took 13 us at any T up to 512.
-constexpr int NORM_THREADS = 1024;
 __device__ __forceinline__ float norm_scale(double s, int K, float eps, double* part, int nwave) {
     s = wave_sum_f64(s);
     if ((threadIdx.x & 63) == 0) part[threadIdx.x >> 6] = s;
@@ -516,32 +515,32 @@ __device__ __forceinline__ float norm_scale(double s, int K, float eps, double* 
     const float mean = (float)(S / (double)K);
     return 1.0f / sqrtf(mean + eps);
 }
-template <bool VEC>
-__global__ __launch_bounds__(NORM_THREADS) void rms_norm_kernel(const float* __restrict__ x, int64_t x_tstride, int K,
-                                                                const float* __restrict__ w, float eps,
-                                                                float* __restrict__ y) {
-    __shared__ double part[NORM_THREADS / 64];
+template <bool VEC, int NT>
+__global__ __launch_bounds__(NT) void rms_norm_kernel(const float* __restrict__ x, int64_t x_tstride, int K,
+                                                      const float* __restrict__ w, float eps,
+                                                      float* __restrict__ y) {
+    __shared__ double part[NT / 64];
     const int t = blockIdx.x;
     const float* xr = x + (int64_t)t * x_tstride;
     float* yr = y + (int64_t)t * K;
     double s = 0.0;
     if constexpr (VEC) {
         const float4* x4 = reinterpret_cast<const float4*>(xr);
-        for (int k = threadIdx.x; k < K / 4; k += NORM_THREADS) {
+        for (int k = threadIdx.x; k < K / 4; k += NT) {
             const float4 a = x4[k];
             s += ((double)(a.x * a.x) + (double)(a.y * a.y)) + ((double)(a.z * a.z) + (double)(a.w * a.w));
         }
-        const float scale = norm_scale(s, K, eps, part, NORM_THREADS / 64);
-        for (int k = threadIdx.x; k < K / 4; k += NORM_THREADS) {
+        const float scale = norm_scale(s, K, eps, part, NT / 64);
+        for (int k = threadIdx.x; k < K / 4; k += NT) {
             const float4 a = x4[k], b = reinterpret_cast<const float4*>(w)[k];
             reinterpret_cast<float4*>(yr)[k] =
                 make_float4(a.x * scale * b.x, a.y * scale * b.y, a.z * scale * b.z, a.w * scale * b.w);
         }
     } else {
 #pragma unroll 4
-        for (int k = threadIdx.x; k < K; k += NORM_THREADS) s += (double)(xr[k] * xr[k]);
-        const float scale = norm_scale(s, K, eps, part, NORM_THREADS / 64);
-        for (int k = threadIdx.x; k < K; k += NORM_THREADS) yr[k] = xr[k] * scale * w[k];
+        for (int k = threadIdx.x; k < K; k += NT) s += (double)(xr[k] * xr[k]);
+        const float scale = norm_scale(s, K, eps, part, NT / 64);
+        for (int k = threadIdx.x; k < K; k += NT) yr[k] = xr[k] * scale * w[k];
     }
 }
 
@@ -623,8 +622,20 @@ hipError_t launch_rms_norm(const float* x, int64_t x_tstride, int T, int K, cons
                            hipStream_t st) {
     if (T <= 0) return hipSuccess;
     const bool vec = K % 4 == 0 && x_tstride % 4 == 0 && (((uintptr_t)x | (uintptr_t)w | (uintptr_t)y) & 15) == 0;
-    hipLaunchKernelGGL(vec ? rms_norm_kernel<true> : rms_norm_kernel<false>, dim3(T), dim3(NORM_THREADS), 0, st, x,
-                       x_tstride, K, w, eps, y);
+    const auto go = [&](auto kernel, int nt) {
+        hipLaunchKernelGGL(kernel, dim3(T), dim3(nt), 0, st, x, x_tstride, K, w, eps, y);
+    };
+    // Threads a row: enough to hold it at four values each, fewer for longer rows,
+    // where a thread keeps several loads in flight; a wider workgroup leaves waves
+    // idle, and many short rows are bound by them. Measured (us, 64 / 256 / 512 /
+    // 1024 threads): 32768 x 128 11.2 / 21.7 / 38.2 / 92.0, 8192 x 1024 14.6 / 13.6 /
+    // 16.3 / 26.8, 128 x 2048 4.2 / 3.1 / 2.8 / 3.0, 2048 x 2048 7.1 / 6.1 / 7.4 / 10.2,
+    // 512 x 4096 7.7 / 4.7 / 4.6 / 5.1, 8192 x 4096 58.3 / 55.5 / 40.7 / 44.6,
+    // 2048 x 8192 32.4 / 30.3 / 28.9 / 24.0; scalar 8192 x 1026 16.6 / 17.1 / 24.8 / 40.8.
+    if (K <= 256) go(vec ? rms_norm_kernel<true, 64> : rms_norm_kernel<false, 64>, 64);
+    else if (K <= 1024 || (K <= 2048 && T >= 1024)) go(vec ? rms_norm_kernel<true, 256> : rms_norm_kernel<false, 256>, 256);
+    else if (K <= 6144) go(vec ? rms_norm_kernel<true, 512> : rms_norm_kernel<false, 512>, 512);
+    else go(vec ? rms_norm_kernel<true, 1024> : rms_norm_kernel<false, 1024>, 1024);
     return hipGetLastError();
 }
 

@@ -140,6 +140,19 @@ def test_rms_norm_misaligned_rows(ctx, oracle):
         np.testing.assert_array_equal(yd.to_host().view(np.uint32), oracle.rms_norm(X, w, EPS).view(np.uint32))
 
 
+@pytest.mark.parametrize("K,T", [(1, 3), (255, 2), (256, 3), (257, 2), (260, 2), (1024, 2), (1025, 2), (1028, 3), (2048, 2),
+                                 (2048, 1024), (2052, 2), (6144, 2), (6148, 2), (6149, 2)])
+def test_rms_norm_row_lengths(ctx, oracle, K, T):
+    """The row lengths where the norm's threads a row change, whole float4s
+    and not: bit for bit the oracle."""
+    from spq4k.hip import DeviceArray
+    X, w = _inputs(np.random.default_rng(K + T), T, K)
+    xd, wd, yd = DeviceArray.from_host(X), DeviceArray.from_host(w), DeviceArray((T, K))
+    ctx.rms_norm_dev(xd.ptr, wd.ptr, EPS, yd.ptr, K, T)
+    ctx.synchronize()
+    np.testing.assert_array_equal(yd.to_host().view(np.uint32), oracle.rms_norm(X, w, EPS).view(np.uint32))
+
+
 @pytest.mark.parametrize("qtype", [TYPE_Q4_K, TYPE_Q5_K, TYPE_Q6_K, TYPE_Q8_0])
 @pytest.mark.parametrize("T,norm", [(1, True), (1, False), (4, True), (12, False)])
 def test_mul_mat_swiglu(ctx, oracle, qtype, T, norm):
