@@ -622,8 +622,12 @@ hipError_t launch_rms_norm(const float* x, int64_t x_tstride, int T, int K, cons
                            hipStream_t st) {
     if (T <= 0) return hipSuccess;
     const bool vec = K % 4 == 0 && x_tstride % 4 == 0 && (((uintptr_t)x | (uintptr_t)w | (uintptr_t)y) & 15) == 0;
+    // a launch holds fewer than 2^32 threads: more rows go in several
+    constexpr int MAX_ROWS = 1 << 21;
     const auto go = [&](auto kernel, int nt) {
-        hipLaunchKernelGGL(kernel, dim3(T), dim3(nt), 0, st, x, x_tstride, K, w, eps, y);
+        for (int t0 = 0; t0 < T; t0 += MAX_ROWS)
+            hipLaunchKernelGGL(kernel, dim3(T - t0 < MAX_ROWS ? T - t0 : MAX_ROWS), dim3(nt), 0, st,
+                               x + (int64_t)t0 * x_tstride, x_tstride, K, w, eps, y + (int64_t)t0 * K);
     };
     // Threads a row: enough to hold it at four values each, fewer for longer rows,
     // where a thread keeps several loads in flight; a wider workgroup leaves waves

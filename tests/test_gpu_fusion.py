@@ -153,6 +153,18 @@ def test_rms_norm_row_lengths(ctx, oracle, K, T):
     np.testing.assert_array_equal(yd.to_host().view(np.uint32), oracle.rms_norm(X, w, EPS).view(np.uint32))
 
 
+def test_rms_norm_many_rows(ctx, oracle):
+    """More rows than one launch of 1024 threads a row could hold (2^32
+    threads), up to the entry's limit of 2^24 rows."""
+    from spq4k.hip import DeviceArray
+    K, T = 2, 1 << 24
+    X, w = _inputs(np.random.default_rng(8), T, K)
+    xd, wd, yd = DeviceArray.from_host(X), DeviceArray.from_host(w), DeviceArray((T, K))
+    ctx.rms_norm_dev(xd.ptr, wd.ptr, EPS, yd.ptr, K, T)
+    ctx.synchronize()
+    np.testing.assert_array_equal(yd.to_host().view(np.uint32), oracle.rms_norm(X, w, EPS).view(np.uint32))
+
+
 @pytest.mark.parametrize("qtype", [TYPE_Q4_K, TYPE_Q5_K, TYPE_Q6_K, TYPE_Q8_0])
 @pytest.mark.parametrize("T,norm", [(1, True), (1, False), (4, True), (12, False)])
 def test_mul_mat_swiglu(ctx, oracle, qtype, T, norm):
