@@ -82,7 +82,7 @@ int         spq4k_synchronize(spq4k_ctx *ctx);
 const char *spq4k_last_error(const spq4k_ctx *ctx);
 int         spq4k_device_count(void);
 /* Grow the context's scratch to at least scratch_bytes (activation planes,
- * K-split partial sums, MoE routing) and its fusion scratch to at least
+ * MoE routing) and its fusion scratch to at least
  * fusion_bytes (normalised rows and gate / up outputs of the unfused
  * spq4k_mul_mat_rms_norm / spq4k_mul_mat_swiglu paths), as the CUDA backend's
  * memory pool grows on demand (ggml_cuda_pool_leg::alloc,
@@ -92,8 +92,8 @@ int         spq4k_device_count(void);
  * before capturing. Buffers replaced by larger ones stay allocated until
  * spq4k_free, so graphs captured earlier stay valid. Sizes: activation
  * planes take 340 bytes per 256 values of each input row (Q8_0: 36 bytes per
- * 32), a K split up to 8 MiB of partial sums beside them; the fusion scratch
- * takes 4 bytes per input value (the norm) plus 8 per output (SwiGLU). */
+ * 32); the partial sums of a K split have 8 MiB of their own; the fusion
+ * scratch takes 4 bytes per input value (the norm) plus 8 per output (SwiGLU). */
 int         spq4k_reserve(spq4k_ctx *ctx, size_t scratch_bytes, size_t fusion_bytes);
 
 /* ---- weights -----------------------------------------------------------

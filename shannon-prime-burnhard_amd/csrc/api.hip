@@ -24,24 +24,16 @@
 
 using namespace spq4k;
 
-// The partial-sum plane of a K-split matmul is held to a fixed budget, so the
-// split (and with it the order of the fp32 sums) depends on the shape alone:
-// not on how much scratch a context happens to hold, and not on whether the
-// call runs on the no-allocation scratch (whose activation planes leave it
-// exactly this much, SPQ4K_NOALLOC_SCRATCH_BYTES - SPQ4K_NOALLOC_PLANES_MAX).
+// The partial-sum plane of a K-split matmul has a buffer of its own and of
+// this size in every context (and behind the activation planes in the
+// no-allocation array), so the split, and with it the order of the fp32 sums,
+// depends on the shape alone: not on how much scratch a context happens to
+// hold, nor on which scratch the call runs on. Inside a scratch of 16 MiB the
+// plane would have to shrink beside planes of 8 to 16 MiB: Q6_K 1024 x 12288 at
+// T = 700 took 86.6 us with what was left against 69.9 with its 8 MiB.
 constexpr size_t KSPLIT_PARTIAL_BYTES = (size_t)8 << 20;
 static_assert(SPQ4K_NOALLOC_SCRATCH_BYTES - SPQ4K_NOALLOC_PLANES_MAX == KSPLIT_PARTIAL_BYTES,
               "the no-allocation scratch leaves a K split its whole budget");
-// Scratch a context starts with. A matmul whose planes fit it splits K only as
-// far as the partial plane fits beside them, so that its call never grows a
-// fresh context's scratch (which a call under capture may not do).
-constexpr size_t INITIAL_SCRATCH_BYTES = (size_t)16 << 20;
-constexpr size_t ksplit_budget(size_t planes) {
-    return planes >= INITIAL_SCRATCH_BYTES || INITIAL_SCRATCH_BYTES - planes >= KSPLIT_PARTIAL_BYTES
-               ? KSPLIT_PARTIAL_BYTES
-               : INITIAL_SCRATCH_BYTES - planes;
-}
-
 
 struct spq4k_ctx {
     int device = 0;
@@ -52,6 +44,7 @@ struct spq4k_ctx {
     // generic device scratch (Q8_K activations, routing tables)
     uint8_t* scratch = nullptr;
     size_t scratch_cap = 0;
+    uint8_t* partial = nullptr;  // partial sums of a K split, KSPLIT_PARTIAL_BYTES
     // intermediates of the fused entry points (normalised rows, gate / up outputs)
     uint8_t* scratch2 = nullptr;
     size_t scratch2_cap = 0;
@@ -244,11 +237,10 @@ struct Around {
     bool glu_done = false;
 };
 
-// extra: bytes of scratch wanted behind the planes (at q8_planes_bytes)
 int q8_planes(spq4k_ctx* c, const float* x, int64_t x_tstride, int T, int nb, Q8Planes* Q, bool perm = false,
-              size_t extra = 0, const Norm* norm = nullptr) {
+              const Norm* norm = nullptr) {
     const size_t items = (size_t)T * nb;
-    int rc = ensure_scratch(c, q8_planes_bytes(T, nb) + extra);
+    int rc = ensure_scratch(c, q8_planes_bytes(T, nb));
     if (rc) return rc;
     int8_t* qs = (int8_t*)c->scratch;
     uint8_t* mn = c->scratch + items * 256;
@@ -394,8 +386,7 @@ int q80_grid(const spq4k_ctx* c, int64_t rows, int nb, int64_t xrows) {
 // tokens a launch as LDS holds (at most 8); a row too long for LDS reads its
 // one token from the planes directly.
 // Q8_0 batches on the matrix cores (gemm_ring_kernel, F = 3): the Q8_0
-// planes of X in the scratch with the partial plane of a K split behind them,
-// then the ring launch (and the reduction of the K ranges).
+// planes of X in the scratch, then the ring launch (and the reduction of the K ranges).
 int q80_gemm(spq4k_ctx* c, int n, const spq4k_weights* const* W, const float* X, float* const* Y, int64_t T) {
     const int64_t K = W[0]->K;
     const int nb = (int)(K / SPQ4K_QK8_0);
@@ -418,19 +409,18 @@ int q80_gemm(spq4k_ctx* c, int n, const spq4k_weights* const* W, const float* X,
     p.fmt = WF_Q80;
     if ((rows + 15) / 16 * ((T + 15) / 16) > (1ll << 31) - 1 || rows > (1ll << 31) - 1)
         return set_err(c, -EINVAL, "gemm: grid too large");
-    const size_t planes = q80_planes_bytes(T, nb);
-    const GemmPlan g = gemm_plan(p, c->num_cus, ksplit_budget(planes));
+    const GemmPlan g = gemm_plan(p, c->num_cus, KSPLIT_PARTIAL_BYTES);
     p.cfg = g.cfg;
     p.ksplit = g.ksplit;
     p.kchunk = g.kchunk;
     Q80Params qp;
     memset(&qp, 0, sizeof qp);
-    int rc = q80_planes(c, X, K, T, nb, &qp, g.partial_bytes);
+    int rc = q80_planes(c, X, K, T, nb, &qp);
     if (rc) return rc;
     p.Q.qs = qp.Aq;
     p.Q.d = qp.Ad;
     p.Q.mn = reinterpret_cast<const uint8_t*>(qp.Aq);   // no min-term plane: a valid address for stray reads
-    p.P = g.ksplit > 1 ? reinterpret_cast<float*>(c->scratch + planes) : nullptr;
+    p.P = g.ksplit > 1 ? reinterpret_cast<float*>(c->partial) : nullptr;
     const hipError_t e = launch_gemm(p, c->stream);
     if (e != hipSuccess) return hip_fail(c, e, "gemm (Q8_0) launch");
     return 0;
@@ -609,7 +599,7 @@ int gemv_launch(spq4k_ctx* c, int n, const spq4k_weights* const* W, const float*
     if (c->preq_mode == 2) preq = false;
     if (around && around->norm) preq = true;
     if (preq) {
-        int rc = q8_planes(c, x, K, (int)T, p.nb, &p.Q, false, 0, around ? around->norm : nullptr);
+        int rc = q8_planes(c, x, K, (int)T, p.nb, &p.Q, false, around ? around->norm : nullptr);
         if (rc) return rc;
     }
     hipError_t e = launch_gemv(p, (int)T, bpr, (int)tiles, c->stream);
@@ -654,7 +644,7 @@ int gemv_chunked(spq4k_ctx* c, int n, const spq4k_weights* const* W, const float
     const int cb_max = LDS_BUDGET / (SPQ4K_GEMV_MAX_T * 292);
     p.chunk_blocks = nb < cb_max ? nb : cb_max;
     Q8Planes Q;
-    int rc = q8_planes(c, X, K, (int)T, nb, &Q, false, 0, norm);
+    int rc = q8_planes(c, X, K, (int)T, nb, &Q, false, norm);
     if (rc) return rc;
     for (int64_t t0 = 0; t0 < T; t0 += SPQ4K_GEMV_MAX_T) {
         const int tc = (int)(T - t0 < SPQ4K_GEMV_MAX_T ? T - t0 : SPQ4K_GEMV_MAX_T);
@@ -799,7 +789,8 @@ int spq4k_init(int device, spq4k_ctx** out) {
     (void)noalloc_scratch_setup(device);
     // scratch for Q8_K activation planes: sized for prefill batches up front
     // so that steady-state calls (and graph capture) never allocate
-    if (ensure_scratch(c, INITIAL_SCRATCH_BYTES) != 0 || ensure_scratch2(c, (size_t)4 << 20) != 0) {
+    if (ensure_scratch(c, (size_t)16 << 20) != 0 || ensure_scratch2(c, (size_t)4 << 20) != 0 ||
+        hipMalloc((void**)&c->partial, KSPLIT_PARTIAL_BYTES) != hipSuccess) {
         if (c->scratch) (void)hipFree(c->scratch);
         if (c->scratch2) (void)hipFree(c->scratch2);
         (void)hipStreamDestroy(c->own_stream);
@@ -816,6 +807,7 @@ void spq4k_free(spq4k_ctx* c) {
     if (c->stream) (void)hipStreamSynchronize(c->stream);
     if (c->scratch) (void)hipFree(c->scratch);
     if (c->scratch2) (void)hipFree(c->scratch2);
+    if (c->partial) (void)hipFree(c->partial);
     for (void* p : c->retired) (void)hipFree(p);
     if (c->own_stream) (void)hipStreamDestroy(c->own_stream);
     delete c;
@@ -1247,8 +1239,7 @@ int spq4k_gemv_multi(spq4k_ctx* c, int n, const spq4k_weights* const* W, const f
 namespace {
 
 // Matrix-core matmul of n matrices sharing the input (shapes checked by the
-// callers): plan, quantise X once into the context scratch (with the partial
-// plane of a K split behind it), launch.
+// callers): plan, quantise X once into the context scratch, launch.
 int gemm_segments(spq4k_ctx* c, int n, const spq4k_weights* const* W, const float* X, float* const* Y, int64_t T,
                   int mode, Around* around) {
     const Norm* norm = around ? around->norm : nullptr;
@@ -1282,21 +1273,20 @@ int gemm_segments(spq4k_ctx* c, int n, const spq4k_weights* const* W, const floa
     }
     hipError_t e;
     if (gemm_use_skinny(p, tiles16)) {
-        int rc = q8_planes(c, X, K, (int)T, p.nb, &p.Q, false, 0, norm);
+        int rc = q8_planes(c, X, K, (int)T, p.nb, &p.Q, false, norm);
         if (rc) return rc;
         p.total_tiles = (int32_t)tiles16;
         e = launch_gemm_skinny(p, c->stream);
         if (e != hipSuccess) return hip_fail(c, e, "gemm skinny launch");
         return 0;
     }
-    const size_t planes = q8_planes_bytes((int)T, p.nb);
-    const GemmPlan g = gemm_plan(p, c->num_cus, ksplit_budget(planes));
+    const GemmPlan g = gemm_plan(p, c->num_cus, KSPLIT_PARTIAL_BYTES);
     p.cfg = g.cfg;
     p.ksplit = g.ksplit;
     p.kchunk = g.kchunk;
-    int rc = q8_planes(c, X, K, (int)T, p.nb, &p.Q, g.perm, g.partial_bytes, norm);
+    int rc = q8_planes(c, X, K, (int)T, p.nb, &p.Q, g.perm, norm);
     if (rc) return rc;
-    p.P = g.ksplit > 1 ? reinterpret_cast<float*>(c->scratch + planes) : nullptr;
+    p.P = g.ksplit > 1 ? reinterpret_cast<float*>(c->partial) : nullptr;
     if (around && around->glu) {
         p.glu = around->glu;
         around->glu_done = true;
@@ -1368,12 +1358,15 @@ int spq4k_mul_mat_noalloc(spq4k_ctx* c, const spq4k_weights* W, const float* X, 
                        "%zu the no-allocation scratch holds for them", (long long)T, (long long)W->K, planes,
                        (size_t)SPQ4K_NOALLOC_PLANES_MAX);
     uint8_t* const own = c->scratch;
+    uint8_t* const own_partial = c->partial;
     const size_t own_cap = c->scratch_cap;
     c->scratch = base;
-    c->scratch_cap = SPQ4K_NOALLOC_SCRATCH_BYTES;
+    c->partial = base + SPQ4K_NOALLOC_PLANES_MAX;
+    c->scratch_cap = SPQ4K_NOALLOC_PLANES_MAX;
     c->no_alloc = true;
     rc = spq4k_mul_mat(c, W, X, Y, T);
     c->scratch = own;
+    c->partial = own_partial;
     c->scratch_cap = own_cap;
     c->no_alloc = false;
     return rc;

@@ -885,7 +885,6 @@ GemmPlan gemm_plan(const GemmParams& p, int num_cus, size_t max_partial_bytes) {
         }
     }
     g.perm = kTiled[g.cfg].ring;
-    g.partial_bytes = g.ksplit > 1 ? (size_t)g.ksplit * per_split : 0;
     return g;
 }
 

@@ -198,12 +198,12 @@ struct GemmParams {
     float* glu;
 };
 // Launch plan of the tiled / ring kernels for a GemmParams (T, nb, segments,
-// cfg): shape, K split and the scratch the partial plane needs.
+// cfg): shape and K split (its partial plane, ksplit * T * rows * 4 bytes, within
+// gemm_plan's max_partial_bytes).
 struct GemmPlan {
     int cfg;
     int ksplit, kchunk;
     bool perm;                 // reads the permuted Q8_K values
-    size_t partial_bytes;      // ksplit * T * rows * 4 when ksplit > 1
 };
 // whether the matmul takes the skinny kernel (16-row tiles: tiles16 of them over all segments)
 bool gemm_use_skinny(const GemmParams& p, int64_t tiles16);

@@ -89,3 +89,40 @@ def test_growth_during_capture_is_refused(oracle):
             _check_sample(oracle, W, Xb, b["yb"].to_host(), "large call captured after spq4k_reserve")
     finally:
         c.close()
+
+
+def test_k_split_beside_large_planes(oracle):
+    """Activation planes of 8 to 16 MiB (700 rows of 48 blocks, 10.9 MiB) do
+    not shrink a K split's room: on a fresh context the call is captured as
+    planes, matmul and the pass that sums the K ranges, its replays match the
+    oracle on sampled tokens and the no-allocation call bit for bit."""
+    import ctypes as C
+
+    import spq4k
+    from spq4k.hip import DeviceArray, Graph, _lib, check
+    m, k, T = 1024, 12288, 700
+    c = spq4k.Context(0)
+    try:
+        rng = np.random.default_rng(14)
+        W = oracle.quantize(14, (rng.standard_normal((m, k)) * 0.02).astype(np.float32))   # Q6_K
+        X = rng.standard_normal((T, k)).astype(np.float32)
+        Wd = c.upload(W, m, k, type=14)
+        xd, yd, y2 = DeviceArray.from_host(X), DeviceArray((T, m)), DeviceArray((T, m))
+        with Graph.capture(c.stream) as g:
+            c.mul_mat_dev(Wd, xd.ptr, yd.ptr, T)
+        n = C.c_size_t()
+        check(_lib().hipGraphGetNodes(C.c_void_p(g.graph), None, C.byref(n)), "hipGraphGetNodes")
+        assert n.value == 3, f"{n.value} launches: K is not split"
+        assert c.lib.spq4k_mul_mat_noalloc(c.handle, Wd.handle, xd.ptr, y2.ptr, T) == 0
+        idx = np.r_[0:4, T - 4:T]
+        exp = oracle.mul_mat_type(14, W, m, k, np.ascontiguousarray(X[idx]))
+        for _ in range(2):
+            yd.fill_byte(0xFF)
+            g.launch()
+            c.synchronize()
+            got = yd.to_host()
+            ok = close_enough(got[idx], exp)
+            assert ok.all(), f"{int((~ok).sum())}/{ok.size} outside tolerance"
+            np.testing.assert_array_equal(got.view(np.uint32), y2.to_host().view(np.uint32))
+    finally:
+        c.close()
