@@ -588,7 +588,7 @@ int gemv_launch(spq4k_ctx* c, int n, const spq4k_weights* const* W, const float*
         !(p.fmt != WF_Q4K && c->gemm_mode == 1)) {
         // 4 <= T <= 8: the sdot4 kernel's integer work grows with T while the
         // matrix cores' 16-token tile costs the same from T = 1 to 16
-        return gemm_segments(c, n, W, x, y, T, c->gemm_mode == 1 ? 1 : 0, around);
+        return gemm_segments(c, n, W, x, y, T, c->gemm_mode, around);
     }
     const int cb_max = LDS_BUDGET / ((int)T * 292);
     p.chunk_blocks = p.nb < cb_max ? p.nb : cb_max;

@@ -256,3 +256,35 @@ def test_gemm_two_stage_shapes(oracle, cfg):
             _check(got, exp, f"cfg={cfg} M={M} K={K} T={T}", exact)
     finally:
         c.close()
+
+
+@pytest.mark.parametrize("T", [5, 12])
+def test_gemm_mode_tiled_small_batch(oracle, T):
+    """SPQ4K_GEMM_MODE=2 keeps a small Q4_K matrix, which would take the skinny
+    kernel, on the tiled kernels at every batch size: planes, matmul and the
+    pass that sums the K ranges (the skinny kernel needs no third launch)."""
+    import ctypes as C
+
+    from _envctx import context_with
+    from spq4k.hip import DeviceArray, Graph, _lib, check
+    M, K = 4096, 2048
+    rng = np.random.default_rng(T)
+    W = oracle.quantize(12, (rng.standard_normal((M, K)) * 0.02).astype(np.float32))
+    X = rng.standard_normal((T, K)).astype(np.float32)
+    launches = []
+    for mode in (0, 2):
+        c = context_with({"SPQ4K_GEMM_MODE": mode})
+        try:
+            Wd = c.upload(W, M, K)
+            xd, yd = DeviceArray.from_host(X), DeviceArray((T, M))
+            with Graph.capture(c.stream) as g:
+                c.mul_mat_dev(Wd, xd.ptr, yd.ptr, T)
+            n = C.c_size_t()
+            check(_lib().hipGraphGetNodes(C.c_void_p(g.graph), None, C.byref(n)), "hipGraphGetNodes")
+            launches.append(n.value)
+            g.launch()
+            c.synchronize()
+            _check(yd.to_host(), oracle.mul_mat_type(12, W, M, K, X), f"mode {mode} T={T}")
+        finally:
+            c.close()
+    assert launches == [2, 3], launches
