@@ -1529,9 +1529,15 @@ int mul_mat_n(spq4k_ctx* c, int n, const spq4k_weights* const* W, const float* X
 }
 
 // Whether a batch's norm runs in the pass that makes the activation planes:
-// K-quant weights (every path of theirs above one token reads Q8_K planes).
+// K-quant weights (every path of theirs above one token reads Q8_K planes),
+// except two or three tokens of at most eight blocks, where the matvec
+// quantises the normalised rows itself for less than the planes cost (us,
+// norm pass and matvec / planes with the norm and matvec, T = 3: 1024 x 1024
+// Q4_K 6.0 / 7.5, 9728 x 2048 11.2 / 11.7, gate and up of 2048 x 2048 Q6_K
+// 10.9 / 11.7; at 3072 values 9728 rows 15.0 / 14.3, gate and up 13.6 / 13.3).
 // Q8_0 batches and one token outside the decode kernel keep the norm pass.
 bool norm_in_planes(const spq4k_ctx* c, const spq4k_weights* W, int64_t T) {
+    if (T < c->gemv_mfma_min_t && W->K <= 8 * SPQ4K_QK_K) return false;
     return T > 1 && W->fmt != WF_Q80 && c->preq_mode != 2;
 }
 
