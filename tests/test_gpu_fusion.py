@@ -87,10 +87,10 @@ def test_mul_mat_rms_norm(ctx, oracle, qtype, T):
         np.testing.assert_array_equal(a.to_host().view(np.uint32), b.to_host().view(np.uint32))
 
 
-@pytest.mark.parametrize("K,T", [(256, 2), (2048, 3), (2304, 3), (2048, 4), (4096, 5), (4352, 3), (16384, 2), (16640, 3), (32768, 2), (33024, 3)])
+@pytest.mark.parametrize("K,T", [(256, 2), (256, 5), (1024, 4), (1280, 4), (2048, 3), (2304, 3), (2048, 4), (4096, 5), (4352, 3), (16384, 2), (16640, 3), (32768, 2), (33024, 3)])
 def test_norm_in_planes(ctx, oracle, K, T):
     """The norm inside the planes pass at the row lengths where its launch
-    shape changes (one pass of 256 / 512 / 1024 threads, two, and the rows read
+    shape changes (one pass of 64 / 256 / 512 / 1024 threads, two, and the rows read
     twice), matvec (T = 2, 3; the norm pass up to 2048 values) and matrix-core
     (T = 4, 5) batches: the same bits, for these inputs, as the norm pass and the
     matmul run one after the other (the two sum the squares in double in another
