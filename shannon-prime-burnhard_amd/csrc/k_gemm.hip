@@ -22,6 +22,7 @@
 //     that fp16 / fp32 represent exactly, so M is exact;
 //   - per super-block acc += d8 (d I - dmin M) in fp32.
 #include "gemv_core.h"
+#include "gemm_plan.h"
 #include "launch.h"
 #include "q6k_core.h"
 #include "ring_core.h"
@@ -500,7 +501,6 @@ __global__ __launch_bounds__(NW * 64) void gemm_ring_kernel(GemmParams p) {
 
 // Sum over the K ranges, in range order, of element i of the partial plane
 // (n elements a range): every range's load issued before the sums.
-constexpr int REDUCE_MAX_SPLIT = 32;
 __device__ __forceinline__ float reduce_ranges(const float* __restrict__ P, int64_t n, int64_t i, int ks) {
     float part[REDUCE_MAX_SPLIT];
 #pragma unroll
@@ -752,7 +752,7 @@ static hipError_t launch_ring_(const GemmParams& p, int grid, hipStream_t st) {
     hipLaunchKernelGGL((gemm_ring_kernel<RT, CT, NW, S, TW, F>), dim3((unsigned)grid), dim3(NW * 64), 0, st, p);
     return hipGetLastError();
 }
-static const TiledShape kTiled[] = {
+static constexpr TiledShape kTiled[] = {
     {256, 64, true, launch_ring_<2, 4, 8, 2>},      // 0: ring 16x16, 8 waves, 2 stages
     {128, 64, true, launch_ring_<1, 4, 8, 3>},      // 1: ring, 8 waves, 3 stages
     {128, 64, true, launch_ring_<2, 4, 4, 3>},      // 2: ring, 4 waves, 3 stages
@@ -808,82 +808,42 @@ constexpr int N_TILED = (int)(sizeof(kTiled) / sizeof(kTiled[0]));
 
 int gemm_tiled_shapes() { return N_TILED; }
 
-static int64_t row_tiles(const GemmParams& p, int rows) {
-    int64_t tiles = 0;
-    for (int i = 0; i < p.nseg; ++i) tiles += (p.seg[i].M + rows - 1) / rows;
-    return tiles;
+// the planner's costs name shapes of their format, with their tiles
+template <int N>
+constexpr bool costs_match(const ShapeCost (&cost)[N], int fmt) {
+    for (const ShapeCost& c : cost)
+        if (c.cfg < 0 || c.cfg >= N_TILED || kTiled[c.cfg].fmt != fmt || !kTiled[c.cfg].ring ||
+            kTiled[c.cfg].rows != c.rows || kTiled[c.cfg].tok != c.tok)
+            return false;
+    return true;
 }
+static_assert(costs_match(kCostQ4K, WF_Q4K) && costs_match(kCostQ6K, WF_Q6K) && costs_match(kCostQ5K, WF_Q5K) &&
+                  costs_match(kCostQ80, WF_Q80),
+              "a planner cost differs from its launch shape");
 
-// What a launch shape costs, measured on an MI355X (256 CUs, cold weights, one
-// K range, 8 and 24 super-blocks a row; us): `t1`, a super-block's step of a
-// launch with one workgroup a CU; `tn`, of one with `occ` workgroups a CU (as
-// many as its LDS leaves room for). Shapes that no size prefers are not listed.
-struct ShapeCost {
-    int cfg, occ;
-    float t1, tn;
-};
-static const ShapeCost kCostQ4K[] = {{8, 3, 0.60f, 1.45f}, {6, 2, 0.90f, 1.86f}, {7, 1, 1.15f, 1.15f},
-                                     {1, 1, 1.70f, 1.70f}, {32, 2, 1.76f, 3.14f}, {11, 1, 3.13f, 3.13f},
-                                     {37, 4, 0.80f, 2.54f}, {33, 2, 1.08f, 1.76f}};
-static const ShapeCost kCostQ6K[] = {{29, 2, 0.92f, 1.57f}, {18, 1, 1.65f, 1.65f}, {16, 1, 1.79f, 1.79f},
-                                     {14, 1, 2.20f, 2.20f}, {17, 1, 4.66f, 4.66f}, {38, 2, 1.15f, 1.92f},
-                                     {34, 2, 1.57f, 2.27f}};
-static const ShapeCost kCostQ5K[] = {{30, 2, 0.80f, 1.28f}, {20, 1, 1.21f, 1.21f}, {23, 1, 1.34f, 1.34f},
-                                     {21, 1, 1.60f, 1.60f}, {19, 1, 2.19f, 2.19f}, {39, 3, 0.94f, 2.25f},
-                                     {35, 2, 1.37f, 2.33f}};
-static const ShapeCost kCostQ80[] = {{31, 2, 1.40f, 1.74f}, {28, 2, 2.21f, 3.24f}, {27, 1, 3.37f, 3.37f},
-                                     {26, 1, 4.23f, 4.23f}, {40, 2, 1.83f, 2.01f}, {36, 2, 3.31f, 3.54f}};
-
-// The launch shape and K split of least estimated time. A launch runs in
-// rounds of occ workgroups a CU; a round costs its fill and drain (4 us: the
-// 512-tile runs of the sweep above against the 256-tile ones) and a step a
-// super-block, the last round less when it leaves CUs (or their second place)
-// empty; a K split adds the reduction pass (3 us and its bytes at 3.5 TB/s). So
-// a grid a little over a whole number of rounds takes fewer ranges or another
-// tile instead: 4096 x 12288 Q6_K at T = 100 ran 320 workgroups, one a CU, in
-// two rounds of ten super-blocks; four ranges make one of twelve.
 GemmPlan gemm_plan(const GemmParams& p, int num_cus, size_t max_partial_bytes) {
-    const ShapeCost* cost = p.fmt == WF_Q6K ? kCostQ6K : p.fmt == WF_Q5K ? kCostQ5K : p.fmt == WF_Q80 ? kCostQ80 : kCostQ4K;
-    const int ncost = (int)(p.fmt == WF_Q6K   ? sizeof kCostQ6K
-                            : p.fmt == WF_Q5K ? sizeof kCostQ5K
-                            : p.fmt == WF_Q80 ? sizeof kCostQ80 : sizeof kCostQ4K) / (int)sizeof(ShapeCost);
-    const bool forced = p.cfg >= 0 && p.cfg < N_TILED && kTiled[p.cfg].fmt == p.fmt;   // not a shape of another format
-    const size_t per_split = (size_t)p.T * p.rows * sizeof(float);
-    int most = max_partial_bytes / per_split < REDUCE_MAX_SPLIT ? (int)(max_partial_bytes / per_split) : REDUCE_MAX_SPLIT;
-    if (most < 1) most = 1;
-
-    GemmPlan g;
-    g.cfg = -1;
-    float best = 0.0f;
-    for (int k = 0; k < (forced ? 1 : ncost); ++k) {
-        ShapeCost c = cost[k];
-        if (forced) {   // its cost if it is listed, else any: only the split is chosen
-            c = {p.cfg, 1, 1.0f, 1.0f};
-            for (int m = 0; m < ncost; ++m)
-                if (cost[m].cfg == p.cfg) c = cost[m];
-        }
-        const TiledShape& s = kTiled[c.cfg];
-        const int64_t tiles = row_tiles(p, s.rows) * ((p.T + s.tok - 1) / s.tok);
-        const int64_t place = (int64_t)num_cus * c.occ;
-        for (int want = 1; want <= (s.ring ? most : 1) && want <= p.nb; ++want) {
-            const int kchunk = (p.nb + want - 1) / want, ks = (p.nb + kchunk - 1) / kchunk;
-            if (ks != want) continue;   // the same ranges as a smaller count
-            const int64_t wgs = tiles * ks, full = wgs / place, rem = wgs - full * place;
-            float step = full * c.tn;
-            if (rem > 0) {   // the fullest CU of the last round sets its pace
-                const int64_t on = (rem + num_cus - 1) / num_cus;
-                step += on == 1 ? c.t1 : c.t1 + (c.tn - c.t1) * (float)(on - 1) / (float)(c.occ - 1);
-            }
-            float us = 4.0f * (float)(full + (rem > 0)) + step * (float)kchunk;
-            if (ks > 1) us += 3.0f + (float)(ks + 1) * (float)per_split / 3.5e6f;
-            if (g.cfg < 0 || us < best) {
-                best = us;
-                g.cfg = c.cfg;
-                g.ksplit = ks;
-                g.kchunk = ks > 1 ? kchunk : p.nb;
-            }
-        }
+    const ShapeCost* cost = kCostQ4K;
+    int ncost = (int)(sizeof kCostQ4K / sizeof(ShapeCost));
+    if (p.fmt == WF_Q6K) cost = kCostQ6K, ncost = (int)(sizeof kCostQ6K / sizeof(ShapeCost));
+    if (p.fmt == WF_Q5K) cost = kCostQ5K, ncost = (int)(sizeof kCostQ5K / sizeof(ShapeCost));
+    if (p.fmt == WF_Q80) cost = kCostQ80, ncost = (int)(sizeof kCostQ80 / sizeof(ShapeCost));
+    ShapeCost one;
+    if (p.cfg >= 0 && p.cfg < N_TILED && kTiled[p.cfg].fmt == p.fmt) {   // forced (not a shape of another format):
+        const TiledShape& s = kTiled[p.cfg];                             // only the split is chosen,
+        one = {p.cfg, s.rows, s.tok, 1, 1.0f, 1.0f};                     // by its cost if it is listed, else any
+        for (int m = 0; m < ncost; ++m)
+            if (cost[m].cfg == p.cfg) one = cost[m];
+        cost = &one;
+        ncost = 1;
+        if (!s.ring) max_partial_bytes = 0;
     }
+    int32_t M[GEMM_MAX_SEG];
+    for (int i = 0; i < p.nseg; ++i) M[i] = p.seg[i].M;
+    const ShapePlan s = plan_shape(cost, ncost, p.nseg, M, p.nb, p.T, num_cus, max_partial_bytes);
+    GemmPlan g;
+    g.cfg = s.cfg;
+    g.ksplit = s.ksplit;
+    g.kchunk = s.kchunk;
     g.perm = kTiled[g.cfg].ring;
     return g;
 }

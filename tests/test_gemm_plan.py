@@ -1,0 +1,111 @@
+"""The matmul planner (csrc/gemm_plan.h, host code) against a direct statement
+of its estimate: every shape, every split, nothing skipped. Host only."""
+import os
+import subprocess
+
+import pytest
+
+REPO = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
+
+DRIVER = r"""
+#include "gemm_plan.h"
+#include <chrono>
+#include <cmath>
+#include <cstdio>
+#include <random>
+#include <set>
+#include <vector>
+using namespace spq4k;
+
+struct Case { int fmt, n, nb; int32_t M[4]; int64_t T; };
+
+static ShapePlan direct(const ShapeCost* cost, int ncost, const Case& c, int cus, size_t room) {
+    int64_t rows = 0;
+    for (int i = 0; i < c.n; ++i) rows += c.M[i];
+    const size_t plane = (size_t)c.T * rows * 4;
+    ShapePlan best = {-1, 1, c.nb};
+    float least = 0;
+    for (int k = 0; k < ncost; ++k) {
+        const ShapeCost& s = cost[k];
+        int64_t tiles = 0;
+        for (int i = 0; i < c.n; ++i) tiles += (c.M[i] + s.rows - 1) / s.rows;
+        tiles *= (c.T + s.tok - 1) / s.tok;
+        for (int ks = 1; ks <= REDUCE_MAX_SPLIT && ks <= c.nb && (ks == 1 || ks * plane <= room); ++ks) {
+            const int chunk = (c.nb + ks - 1) / ks;
+            if ((c.nb + chunk - 1) / chunk != ks) continue;
+            const int64_t place = (int64_t)cus * s.occ, full = tiles * ks / place, rem = tiles * ks % place;
+            float step = (float)full * s.tn;
+            const int64_t on = (rem + cus - 1) / cus;
+            if (on == 1) step += s.t1;
+            if (on > 1) step += s.t1 + (s.tn - s.t1) * (float)(on - 1) / (float)(s.occ - 1);
+            float us = 4.0f * (float)(full + (rem > 0)) + step * (float)chunk;
+            if (ks > 1) us += 3.0f + (float)(ks + 1) * (float)plane / 3.5e6f;
+            if (best.cfg < 0 || us < least) { least = us; best = {s.cfg, ks, ks > 1 ? chunk : c.nb}; }
+        }
+    }
+    return best;
+}
+
+int main() {
+    const ShapeCost* cost[4] = {kCostQ4K, kCostQ5K, kCostQ6K, kCostQ80};
+    const int ncost[4] = {sizeof kCostQ4K / sizeof(ShapeCost), sizeof kCostQ5K / sizeof(ShapeCost),
+                          sizeof kCostQ6K / sizeof(ShapeCost), sizeof kCostQ80 / sizeof(ShapeCost)};
+    std::mt19937_64 r(1);
+    auto draw = [&](double lo, double hi) {
+        return (int)std::lround(std::exp(std::uniform_real_distribution<>(std::log(lo), std::log(hi))(r)));
+    };
+    std::vector<Case> cases;
+    for (int i = 0; i < 100000; ++i) {
+        Case c = {(int)(r() % 4), r() % 2 ? 1 : 1 + (int)(r() % 4), draw(1, 128), {}, 0};
+        for (int32_t& m : c.M) m = draw(1, 160000);
+        c.T = i % 100 ? draw(1, 5000) : draw(1, 1 << 20);
+        cases.push_back(c);
+    }
+    std::set<int> used;
+    int wrong = 0;
+    for (const Case& c : cases)
+        for (int cus : {256, 64}) {
+            const ShapePlan a = direct(cost[c.fmt], ncost[c.fmt], c, cus, (size_t)8 << 20);
+            const ShapePlan b = plan_shape(cost[c.fmt], ncost[c.fmt], c.n, c.M, c.nb, c.T, cus, (size_t)8 << 20);
+            if (cus == 256) used.insert(b.cfg);
+            if (a.cfg != b.cfg || a.ksplit != b.ksplit || a.kchunk != b.kchunk) ++wrong;
+        }
+    int idle = 0;
+    for (int f = 0; f < 4; ++f)
+        for (int k = 0; k < ncost[f]; ++k) idle += !used.count(cost[f][k].cfg);
+    double best[2] = {1e9, 1e9};
+    volatile int sink = 0;
+    for (int rep = 0; rep < 5; ++rep)
+        for (int which = 0; which < 2; ++which) {
+            const auto t0 = std::chrono::steady_clock::now();
+            for (const Case& c : cases)
+                sink = sink + (which ? plan_shape(cost[c.fmt], ncost[c.fmt], c.n, c.M, c.nb, c.T, 256, (size_t)8 << 20)
+                                     : direct(cost[c.fmt], ncost[c.fmt], c, 256, (size_t)8 << 20)).ksplit;
+            const double s = std::chrono::duration<double>(std::chrono::steady_clock::now() - t0).count();
+            if (s < best[which]) best[which] = s;
+        }
+    printf("%d %d %.3f %.0f\n", wrong, idle, best[1] / best[0], best[1] / cases.size() * 1e9);
+}
+"""
+
+
+@pytest.fixture(scope="module")
+def result(tmp_path_factory):
+    d = tmp_path_factory.mktemp("plan")
+    src, exe = str(d / "plan.cpp"), str(d / "plan")
+    open(src, "w").write(DRIVER)
+    subprocess.run(["g++", "-O2", "-std=c++17", "-ffp-contract=off", "-Wall", "-Werror", "-I",
+                    os.path.join(REPO, "shannon-prime-burnhard_amd", "csrc"), src, "-o", exe], check=True)
+    out = subprocess.run([exe], check=True, capture_output=True, text=True).stdout.split()
+    return int(out[0]), int(out[1]), float(out[2]), float(out[3])
+
+
+def test_plans_are_the_least_estimates(result):
+    """100,000 drawn matmuls on 256 and 64 CUs: shape, split and range length."""
+    assert result[0] == 0
+
+
+def test_plan_skips_what_cannot_win(result):
+    """A call's planning on the host takes less than pricing every split (about
+    0.55 of it; 0.85 leaves room for a loaded machine)."""
+    assert result[2] < 0.85, result
