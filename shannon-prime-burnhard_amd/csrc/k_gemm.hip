@@ -809,37 +809,34 @@ constexpr int N_TILED = (int)(sizeof(kTiled) / sizeof(kTiled[0]));
 int gemm_tiled_shapes() { return N_TILED; }
 
 // the planner's costs name shapes of their format, with their tiles
-template <int N>
-constexpr bool costs_match(const ShapeCost (&cost)[N], int fmt) {
-    for (const ShapeCost& c : cost)
+constexpr bool costs_match(const PlanCosts& p, int fmt) {
+    for (int k = 0; k < p.n; ++k) {
+        const ShapeCost& c = p.shape[k];
         if (c.cfg < 0 || c.cfg >= N_TILED || kTiled[c.cfg].fmt != fmt || !kTiled[c.cfg].ring ||
             kTiled[c.cfg].rows != c.rows || kTiled[c.cfg].tok != c.tok)
             return false;
+    }
     return true;
 }
-static_assert(costs_match(kCostQ4K, WF_Q4K) && costs_match(kCostQ6K, WF_Q6K) && costs_match(kCostQ5K, WF_Q5K) &&
-                  costs_match(kCostQ80, WF_Q80),
+static_assert(costs_match(kPlanQ4K, WF_Q4K) && costs_match(kPlanQ6K, WF_Q6K) && costs_match(kPlanQ5K, WF_Q5K) &&
+                  costs_match(kPlanQ80, WF_Q80),
               "a planner cost differs from its launch shape");
 
 GemmPlan gemm_plan(const GemmParams& p, int num_cus, size_t max_partial_bytes) {
-    const ShapeCost* cost = kCostQ4K;
-    int ncost = (int)(sizeof kCostQ4K / sizeof(ShapeCost));
-    if (p.fmt == WF_Q6K) cost = kCostQ6K, ncost = (int)(sizeof kCostQ6K / sizeof(ShapeCost));
-    if (p.fmt == WF_Q5K) cost = kCostQ5K, ncost = (int)(sizeof kCostQ5K / sizeof(ShapeCost));
-    if (p.fmt == WF_Q80) cost = kCostQ80, ncost = (int)(sizeof kCostQ80 / sizeof(ShapeCost));
+    PlanCosts costs = p.fmt == WF_Q6K ? kPlanQ6K : p.fmt == WF_Q5K ? kPlanQ5K : p.fmt == WF_Q80 ? kPlanQ80 : kPlanQ4K;
     ShapeCost one;
     if (p.cfg >= 0 && p.cfg < N_TILED && kTiled[p.cfg].fmt == p.fmt) {   // forced (not a shape of another format):
         const TiledShape& s = kTiled[p.cfg];                             // only the split is chosen,
-        one = {p.cfg, s.rows, s.tok, 1, 1.0f, 1.0f};                     // by its cost if it is listed, else any
-        for (int m = 0; m < ncost; ++m)
-            if (cost[m].cfg == p.cfg) one = cost[m];
-        cost = &one;
-        ncost = 1;
+        one = {p.cfg, s.rows, s.tok, 1, 4.0f, 1.0f, 1.0f};               // by its cost if it is listed, else any
+        for (int m = 0; m < costs.n; ++m)
+            if (costs.shape[m].cfg == p.cfg) one = costs.shape[m];
+        costs.shape = &one;
+        costs.n = 1;
         if (!s.ring) max_partial_bytes = 0;
     }
     int32_t M[GEMM_MAX_SEG];
     for (int i = 0; i < p.nseg; ++i) M[i] = p.seg[i].M;
-    const ShapePlan s = plan_shape(cost, ncost, p.nseg, M, p.nb, p.T, num_cus, max_partial_bytes);
+    const ShapePlan s = plan_shape(costs, p.nseg, M, p.nb, p.T, num_cus, max_partial_bytes);
     GemmPlan g;
     g.cfg = s.cfg;
     g.ksplit = s.ksplit;
