@@ -134,26 +134,39 @@ size_t type_align(int type) { return type == SPQ4K_TYPE_Q4_K || type == SPQ4K_TY
 bool fmt_has_mfma(int fmt) { return fmt == WF_Q4K || fmt == WF_Q6K || fmt == WF_Q5K; }
 // formats of the expert-gathered ring kernel (moe_ring_kernel)
 bool fmt_has_moe_ring(int fmt) { return fmt == WF_Q4K || fmt == WF_Q6K || fmt == WF_Q5K; }
-// Shape of the expert ring kernel by the pairs an active expert receives on
-// average: 16-pair tiles a workgroup takes at a time (ct) and waves (16 rows
-// each). An expert of more pairs than a workgroup takes is streamed again for
-// the rest; a wider tile holds fewer stages in LDS, so fewer bytes in flight.
-// Measured (us, the routed-expert block of 128 experts, top-8, 2048 -> 768,
-// ct = 1 with 8 waves / ct = 2 / ct = 4 with 4): Q4_K at 6 pairs 103 / 120 /
-// 153, 8 pairs 124 / 123 / 155, 12.5 pairs 158 / 133 / 163; 32 experts at 64
-// pairs 126 / 113 / 108; 60 experts of 3072 -> 1536 at 25 pairs 283 / 285 / 286
-// with 4 waves, and ct = 2 / 4 with 8 waves 248 / 238. Q6_K down bank in the
-// same block (8 waves for ct = 2): 8 pairs 145 / 150, 10 pairs 176 / 152,
-// 32 experts at 32 pairs 96 / 95 / 69. One pair tile, 4 / 8 waves (down bank,
-// T = 32): Q6_K 54.9 / 59.9, Q5_K 45.0 / 48.0, Q4_K (the MoE layer)
-// 97.0 / 88.7, Q8_0 64.2 / 57.4.
+// Shape of the expert ring kernel: 16-pair tiles a workgroup takes at a time (ct)
+// and waves (16 rows each). An expert of more pairs than a workgroup takes is
+// streamed again for the rest, and the launch waits for its fullest expert; a
+// wider tile holds fewer stages in LDS, so fewer bytes in flight. The line
+// therefore lies where an expert in a few receives more than 16 (32) pairs, below
+// that as a mean, the more so the more experts there are. Measured (one bank, uniform
+// routing, us, ct = 1 / 2 / 4 in the waves below): Q4_K 128 experts of 768 x 2048 at
+// 8 pairs 36 / 43 / 54, 10 pairs 42 / 43 / 55, 12 pairs 51 / 44 / 56, 22 pairs 67 /
+// 49 / 60, 25 pairs 72 / 70 / 62; 60 experts of 1536 x 3072 at 11 pairs 46 / 60 / 78,
+// 13 pairs 66 / 61 / 78, 22 pairs 91 / 84 / 81; 8 experts of 14336 x 4096 at 13 pairs
+// 69 / 98 / 124, 18 pairs 103 / 99 / 126, 28 pairs 123 / 102 / 127, 32 pairs 148 / 152 /
+// 127; Q6_K 128 experts at 9 pairs 54 / 67 / 73, 11 pairs 77 / 67 / 73; Q5_K 44 / 51 / 65
+// and 65 / 54 / 66; 60 experts of 1536 x 3072 at 11 / 12 pairs Q6_K 76 / 87 and 107 / 87,
+// Q5_K 61 / 72 and 88 / 72 (ct = 1 / 2). Routing that favours some experts would want
+// the wider tile a few pairs earlier; the host does not see it. Waves, 4 / 8: one
+// tile Q4_K 37 / 36, Q6_K 53 / 65, Q5_K 43 / 50 (128 experts, 8 pairs); two tiles Q4_K
+// 44 / 50, Q6_K 78 / 67 (12 pairs); four Q4_K 62 / 67 (25 pairs), 87 / 86 with 12
+// super-blocks (60 experts, 40 pairs), Q6_K 80 / 89; rows enough for two 128-row tiles
+// a CU in experts of over 2048 rows: Q4_K 3072 x 1536 two tiles 1.21, four 1.30 times as
+// long with 4 waves, 14336 x 4096 1.11 and 1.27, Q6_K four tiles 1.24 and 1.16. Q8_0:
+// one tile (no wider instance is built), 64.2 / 57.4 (down bank, T = 32).
 struct MoeRingShape {
     int ct, waves;
 };
-MoeRingShape moe_ring_shape(const spq4k_ctx* c, int fmt, int64_t mean_pairs, int nb) {
+MoeRingShape moe_ring_shape(const spq4k_ctx* c, int fmt, int64_t mean_pairs, int nb, int64_t M, int64_t max_act) {
+    const int many = max_act > 64 ? 2 : max_act > 16 ? 1 : 0;
+    const int one = (many == 2 ? 9 : many ? 11 : 13) + (fmt == WF_Q4K), two = many == 2 ? 22 : many ? 23 : 27;
+    const bool tall = M > 2048 && M * max_act >= 2 * 128 * (int64_t)c->num_cus;
     MoeRingShape s;
-    s.ct = fmt == WF_Q80 || mean_pairs <= 8 ? 1 : mean_pairs <= 20 ? 2 : 4;
+    s.ct = fmt == WF_Q80 || mean_pairs <= one ? 1 : mean_pairs <= two ? 2 : 4;
     if (s.ct == 1) s.waves = fmt == WF_Q6K || fmt == WF_Q5K ? 4 : 8;
+    else if (fmt == WF_Q5K) s.waves = 4;
+    else if (tall) s.waves = 8;
     else if (s.ct == 2) s.waves = fmt == WF_Q6K ? 8 : 4;
     else s.waves = fmt == WF_Q4K && nb > 8 ? 8 : 4;
     // a forced wave count (SPQ4K_MOE_RING_WAVES) takes the nearest instance
@@ -1463,7 +1476,7 @@ int q80_moe(spq4k_ctx* c, const spq4k_weights* const* banks, int nbank, const in
             mp.bank1 = banks[1]->data;
             mp.Y1 = Ys[1];
         }
-        const int nw = moe_ring_shape(c, WF_Q80, mean_pairs, mp.nb).waves;
+        const int nw = moe_ring_shape(c, WF_Q80, mean_pairs, mp.nb, M, max_act).waves;
         const int64_t ntiles = (M + 16 * nw - 1) / (16 * nw);
         int64_t rtw = ntiles * max_act * nbank / (2 * (int64_t)c->num_cus);
         if (rtw < 1) rtw = 1;
@@ -1819,7 +1832,7 @@ int moe_ring_run(spq4k_ctx* c, const spq4k_weights* const* banks, int nbank, con
     }
     // row tiles a workgroup streams: as many as still leave two workgroups
     // per CU over the experts (of every bank) that can be active
-    const MoeRingShape rs = moe_ring_shape(c, bank->fmt, (n_pairs + max_act - 1) / max_act, nb);
+    const MoeRingShape rs = moe_ring_shape(c, bank->fmt, (n_pairs + max_act - 1) / max_act, nb, M, max_act);
     const int nw = rs.waves;
     p.ring_ct = rs.ct;
     const int64_t ntiles = (M + 16 * nw - 1) / (16 * nw);

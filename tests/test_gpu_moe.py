@@ -119,31 +119,53 @@ def test_moe_paths_agree(oracle, T, ne11, M, K):
         _check(got, exp, f"{env} T={T} ne11={ne11} M={M} K={K}")
 
 
+def _uneven_ids(rng, T, E, k):
+    return np.argsort(-(rng.standard_normal((T, E)) + np.linspace(0, 1.5, E)), axis=1)[:, :k].astype(np.int32)
+
+
 @pytest.mark.parametrize("qtype", [12, 13, 14])   # Q4_K, Q5_K, Q6_K
-@pytest.mark.parametrize("T,K", [(40, 768), (40, 2560), (150, 768), (150, 2560)])
+@pytest.mark.parametrize("T,K", [(60, 768), (60, 2560), (150, 768), (150, 2560)])
 def test_moe_pair_tiles(oracle, qtype, T, K):
-    """Experts of about 13 and 50 pairs, which take two and four 16-pair tiles
+    """Experts of about 20 and 50 pairs, which take two and four 16-pair tiles
     of a workgroup at a time (uneven, some partly empty; ragged rows), short
-    and long rows: element-wise against the oracle, and bit for bit against a
-    forced wave count (the tiles hold the same sums)."""
+    and long rows: element-wise against the oracle, and bit for bit against the
+    same tokens in slices of 20, whose experts take one tile, and against the
+    other wave count where the wide tile has one (Q5_K's has 4 waves only)."""
     from _envctx import context_with
     E, k, M = 6, 2, 147
     rng = np.random.default_rng(qtype + T + K)
     W = oracle.quantize(qtype, (rng.standard_normal((E * M, K)) * 0.02).astype(np.float32))
     X = rng.standard_normal((T, 1, K)).astype(np.float32)
-    ids = np.argsort(-(rng.standard_normal((T, E)) + np.linspace(0, 1.5, E)), axis=1)[:, :k].astype(np.int32)
+    ids = _uneven_ids(rng, T, E, k)
     outs = []
-    for env in ({}, {"SPQ4K_MOE_RING_WAVES": 4}, {"SPQ4K_MOE_RING_WAVES": 8}):
+    for env in ({},) if qtype == 13 else ({}, {"SPQ4K_MOE_RING_WAVES": 4}, {"SPQ4K_MOE_RING_WAVES": 8}):
         c = context_with(env)
         try:
             bank = c.upload(W, M, K, E, type=qtype)
             outs.append(c.mul_mat_id(bank, X, ids))
+            if not env:
+                outs.append(np.concatenate([c.mul_mat_id(bank, X[t:t + 20], ids[t:t + 20]) for t in range(0, T, 20)]))
             bank.free()
         finally:
             c.close()
     _check(outs[0], oracle.mul_mat_id_type(qtype, W, M, K, E, X, ids), f"type {qtype} T={T} K={K}")
     for o in outs[1:]:
         np.testing.assert_array_equal(outs[0].view(np.uint32), o.view(np.uint32))
+
+
+@pytest.mark.parametrize("T", [21, 40, 41, 42, 43, 70, 82, 85])
+def test_moe_pair_tile_lines(ctx, oracle, T):
+    """Mean pairs either side of the lines between one, two and four tiles
+    (E = 6, two of them a token: 7, 14, 14, 14, 15, 24, 28 and 29 pairs)."""
+    E, k, M, K = 6, 2, 80, 512
+    rng = np.random.default_rng(T)
+    for qtype in (12, 13, 14):
+        W = oracle.quantize(qtype, (rng.standard_normal((E * M, K)) * 0.02).astype(np.float32))
+        X = rng.standard_normal((T, 1, K)).astype(np.float32)
+        ids = _uneven_ids(rng, T, E, k)
+        bank = ctx.upload(W, M, K, E, type=qtype)
+        _check(ctx.mul_mat_id(bank, X, ids), oracle.mul_mat_id_type(qtype, W, M, K, E, X, ids), f"type {qtype} T={T}")
+        bank.free()
 
 
 @pytest.mark.parametrize("mode", [0, 2, 3])
