@@ -153,6 +153,37 @@ def test_moe_pair_tiles(oracle, qtype, T, K):
         np.testing.assert_array_equal(outs[0].view(np.uint32), o.view(np.uint32))
 
 
+@pytest.mark.parametrize("qtype", [12, 13, 14])   # Q4_K, Q5_K, Q6_K
+@pytest.mark.parametrize("T", [60, 150])
+def test_moe_pair_tiles_block_forms(ctx, oracle, qtype, T):
+    """The two forms a routed-expert block's prompt batch takes, with two and
+    four pair tiles: gate and up as two banks of one launch, and a down bank
+    with one input row a pair (ne11 = n_used). Each against the oracle, and bit
+    for bit against one bank at a time and slices of 20 tokens (one tile)."""
+    from spq4k.hip import DeviceArray
+    E, k, M, K = 6, 2, 147, 768
+    rng = np.random.default_rng(qtype + T)
+    banks = [oracle.quantize(qtype, (rng.standard_normal((E * M, K)) * 0.02).astype(np.float32)) for _ in range(2)]
+    Wd = [ctx.upload(b, M, K, E, type=qtype) for b in banks]
+    X = rng.standard_normal((T, 1, K)).astype(np.float32)
+    Xp = rng.standard_normal((T, k, K)).astype(np.float32)
+    ids = _uneven_ids(rng, T, E, k)
+    idd, xd, yd = DeviceArray.from_host(ids), DeviceArray.from_host(X), [DeviceArray((T, k, M)) for _ in range(2)]
+    ctx.moe_multi_dev(Wd, idd.ptr, k, 1, T, xd.ptr, [y.ptr for y in yd])
+    ctx.synchronize()
+    down = ctx.mul_mat_id(Wd[0], Xp, ids)
+    for i in range(2):
+        got = yd[i].to_host()
+        _check(got, oracle.mul_mat_id_type(qtype, banks[i], M, K, E, X, ids), f"bank {i} type {qtype} T={T}")
+        one = np.concatenate([ctx.mul_mat_id(Wd[i], X[t:t + 20], ids[t:t + 20]) for t in range(0, T, 20)])
+        np.testing.assert_array_equal(got.view(np.uint32), one.view(np.uint32))
+    _check(down, oracle.mul_mat_id_type(qtype, banks[0], M, K, E, Xp, ids), f"row a pair, type {qtype} T={T}")
+    one = np.concatenate([ctx.mul_mat_id(Wd[0], Xp[t:t + 20], ids[t:t + 20]) for t in range(0, T, 20)])
+    np.testing.assert_array_equal(down.view(np.uint32), one.view(np.uint32))
+    for w in Wd:
+        w.free()
+
+
 @pytest.mark.parametrize("T", [21, 40, 41, 42, 43, 70, 82, 85])
 def test_moe_pair_tile_lines(ctx, oracle, T):
     """Mean pairs either side of the lines between one, two and four tiles

@@ -121,6 +121,32 @@ def test_moe_ffn_30b(ctx, oracle, down_type, T):
         a.free()
 
 
+@pytest.mark.parametrize("down_type", [TYPE_Q4_K, TYPE_Q6_K])
+@pytest.mark.parametrize("T", [60, 150])
+def test_moe_ffn_pair_tiles(ctx, oracle, down_type, T):
+    """Experts of about 20 and 50 pairs (two and four 16-pair tiles of the ring
+    kernel at a time, gate and up in one launch, down with a row a pair): the
+    block equals, bit for bit, its slices of 20 tokens, whose experts take one
+    tile, and the oracle's chain normwise."""
+    E, k, D_, F = 6, 2, 768, 512
+    rng = np.random.default_rng(T + down_type)
+    gate, gh = _bank(ctx, TYPE_Q4_K, E, F, D_, 21)
+    up, uh = _bank(ctx, TYPE_Q4_K, E, F, D_, 22)
+    down, dh = _bank(ctx, down_type, E, D_, F, 23)
+    ids, w = _routing(rng, T, E, k)
+    X = rng.standard_normal((T, D_)).astype(np.float32)
+    Y = ctx.moe_ffn(gate, up, down, ids, w, X)
+    parts = [ctx.moe_ffn(gate, up, down, ids[t:t + 20], w[t:t + 20], X[t:t + 20]) for t in range(0, T, 20)]
+    _bits_equal(Y, np.concatenate(parts), f"T={T} in slices of 20")
+    X3 = X[:, None, :]
+    H = oracle.swiglu(oracle.mul_mat_id(gh, F, D_, E, X3, ids), oracle.mul_mat_id(uh, F, D_, E, X3, ids))
+    Yo = _weighted_sum(_mmid(oracle, down_type, dh, D_, F, E, H, ids), w)
+    err = np.linalg.norm(Y.astype(np.float64) - Yo) / np.linalg.norm(Yo.astype(np.float64))
+    assert err < CHAIN_NORMWISE, f"block T={T} normwise {err:.3e}"
+    for a in (gate, up, down):
+        a.free()
+
+
 @pytest.mark.parametrize("n_ff,n_used,T,down_type", [
     (768, 8, 8, TYPE_Q4_K),      # 64 pairs, the largest small batch
     (768, 8, 9, TYPE_Q4_K),      # 72 pairs: down on the matrix cores, then the combine
