@@ -344,14 +344,17 @@ int spq4k_moe_ffn_host(spq4k_ctx *ctx, const spq4k_weights *gate, const spq4k_we
  *                          launch, the norm in the matvec's prologue;
  *                          otherwise spq4k_mul_mat's path on the normalised
  *                          rows (K-quant weights: the norm in the pass that
- *                          quantises them).
+ *                          quantises them, its squares added in an order of
+ *                          its own, so the rows agree with spq4k_rms_norm's
+ *                          in all but the bits that its note above allows).
  * spq4k_mul_mat_swiglu   : y = silu(Wg . xb) * (Wu . xb), xb = x, or
  *                          rms_norm(x) * norm_w when norm_w is not NULL (the
  *                          dense SwiGLU front half, forward.cpp:1703-1706;
  *                          ggml-cuda fuses the same gate in mmvq.cu:437-470):
  *                          at T = 1 one launch (gate row and up row side by
  *                          side, SiLU and the product in the epilogue);
- *                          otherwise gate and up, then one element-wise pass.
+ *                          otherwise gate and up, then one element-wise pass
+ *                          (where K is split, the pass that sums its ranges).
  *                          Wg and Wu share type, K and M; y is [T][M].
  * Device pointers; x, norm_w 16-byte aligned; eps >= 0. */
 int spq4k_rms_norm(spq4k_ctx *ctx, const float *x, const float *w, float eps, float *y, int64_t K, int64_t T);

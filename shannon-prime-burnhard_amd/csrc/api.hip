@@ -63,7 +63,7 @@ struct spq4k_ctx {
     // bytes than the ring, but skips its prep launch: the 128-expert Q4_K layer
     // takes 49.0 us against 56.5 on the ring
     int moe_dec_max_t = 8;
-    int moe_ring_waves = 0;      // SPQ4K_MOE_RING_WAVES: 4 or 8 waves (64- or 128-row tiles) in the expert ring kernel, 0 by format
+    int moe_ring_waves = 0;      // SPQ4K_MOE_RING_WAVES: 4 or 8 waves (64- or 128-row tiles) in the expert ring kernel, 0 as moe_ring_shape chooses
     int moe_dec_waves = 0;       // SPQ4K_MOE_DEC_WAVES: 8 or 12 waves in a GLU expert sweep, 0 by grid
     uint64_t* dec_stamps = nullptr;   // spq4k_set_decode_stamps: the decode kernel's wave timestamps
     size_t dec_stamps_n = 0;

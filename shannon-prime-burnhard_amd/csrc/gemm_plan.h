@@ -70,8 +70,9 @@ struct ShapePlan {
 // This runs on the host in every matmul call, so the splits and their reduction
 // are worked out once for all shapes, and a split whose bound (one round of
 // `t1` steps) already costs more than the best is not priced: a Q4_K plan of
-// 24576 x 4096 at T = 5 takes 0.37 us against 0.82, of 6144 x 4096 0.26 against
-// 0.84, a Q6_K one of 4096 x 12288 at T = 100 0.20 against 0.33 (2.7 GHz Xeon).
+// 24576 x 4096 at T = 5 takes 0.31 us, of 6144 x 4096 0.24, a Q6_K one of 4096 x
+// 12288 at T = 100 0.16 (2.7 GHz Xeon); all shapes and splits priced one by one,
+// two divisions each, took 0.82, 0.84 and 0.33.
 inline ShapePlan plan_shape(const PlanCosts& p, int n, const int32_t* M, int nb, int64_t T, int num_cus,
                             size_t max_partial_bytes) {
     size_t rows = 0;

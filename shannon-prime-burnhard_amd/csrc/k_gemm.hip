@@ -723,12 +723,16 @@ hipError_t launch_gemm_skinny(const GemmParams& p, hipStream_t st) {
 // The skinny form takes what mode 1 forces, and small Q4_K matrices of at most
 // 16 tokens: its waves' sums meet in LDS, so no reduction launch follows, but
 // every 16 rows read all the activations and its waves wait for their loads
-// once a chunk. Measured (us, at T = 4 / 8 / 16, against the ring and its
-// reduction): 4096 x 2048 6.8 / 7.1 / 7.8 against 9.9 / 10.2 / 10.6,
-// 8192 x 2048 8.6 / 9.2 against 10.0 / 10.1, 4096 x 4096 9.0 / 9.7 / 10.5
-// against 11.3 / 11.4 / 11.9; not 1024 x 4096 (8.6 / 9.3 / 10.3 against
-// 9.4 / 9.3 / 9.7), 6144 x 4096 (12.8 / 14.2 / 16.5 against 13.2 / 13.7 / 14.7)
-// or 4096 x 8192 (12.8 / 14.2 against 13.7 / 14.1).
+// once a chunk. Measured (us at T = 4 / 8 / 12 / 16, skinny against the ring as
+// planned and its reduction): up to 2048 values 512 rows 6.5 / 6.9 / 7.2 / 7.5
+// against 8.3 / 8.4 / 8.5 / 8.6, 4096 rows 7.3 / 7.5 / 7.9 / 8.2 against 10.3 / 10.3 /
+// 10.5 / 10.7, 8192 rows 9.1 / 9.6 / 10.3 / 10.9 against 10.4 / 10.5 / 10.6 / 10.6; up to
+// 4096 values 2048 rows 9.1 / 9.7 / 10.3 / 10.7 against 10.3 / 10.5 / 10.6 / 10.7, 4096
+// rows 9.3 / 9.9 / 10.4 / 10.8 against 11.5 / 11.6 / 11.7 / 11.9 (two of the 16-row
+// workgroups a CU: 5120 rows, a second round, 13.0 / 14.4 / 15.8 / 16.8 against 12.5 /
+// 12.8 / 13.1 / 13.2; 1024 rows leave CUs idle, 9.0 / 9.6 / 10.2 / 10.6 against 9.5 / 9.6 /
+// 9.7 / 9.9). One line for all T: at T = 4 alone 8192 x 4096 (13.5 against 14.4) and
+// 4096 x 8192 (13.4 against 14.5) would gain, at T = 16 they lose 12%.
 bool gemm_use_skinny(const GemmParams& p, int64_t tiles16) {
     if (p.mode == 1) return true;
     if (p.mode != 0 || p.cfg >= 0 || p.fmt != WF_Q4K || p.T > 16) return false;
@@ -792,9 +796,7 @@ static constexpr TiledShape kTiled[] = {
     {128, 64, true, launch_ring_<1, 2, 4, 2, 32>},   // 32: ring 32x32, 4 waves, 2 stages (two workgroups a CU)
     // 64-row tiles, 4 waves, 2 stages: two to four workgroups a CU, so that one's
     // barriers do not hold the others' waves in step and a grid fills its last
-    // round better. A step of two 64 x 64 tiles a CU against one of 128 x 64 (us):
-    // Q8_0 3.54 / 4.23, Q4_K 1.76 / 1.70, Q6_K 2.27 / 2.20, Q5_K 2.33 / 2.19;
-    // 13824 x 5120 Q5_K at T = 150 runs 66.5 us against 86.7 with 128 x 64.
+    // round better: 13824 x 5120 Q5_K at T = 150 runs 66.5 us against 86.7 with 128 x 64.
     {64, 64, true, launch_ring_<1, 4, 4, 2>},                   // 33
     {64, 64, true, launch_ring_<1, 4, 4, 2, 16, 1>, WF_Q6K},    // 34
     {64, 64, true, launch_ring_<1, 4, 4, 2, 16, 2>, WF_Q5K},    // 35

@@ -797,10 +797,11 @@ hipError_t launch_moe_gemv(const MoeParams& p, int tc, int bpr, int grid, hipStr
 // Matrix-core form for batches whose experts receive several pairs.
 //   moe_prep_kernel: workgroup 0 builds the routing tables (route_block), the
 //   others quantise the input rows into permuted Q8_K planes.
-//   moe_ring_kernel: workgroup (a, g) takes active expert a and its 128-row
-//   tiles g*ring_rt .. +ring_rt; the expert's pairs are gathered 16 CT at a time
-//   as the tokens of the LDS ring of gemm_ring_kernel (eight waves, one
-//   16-row tile each, direct global -> LDS loads S - 1 super-blocks ahead)
+//   moe_ring_kernel: workgroup (a, g) takes active expert a and its row tiles
+//   g*ring_rt .. +ring_rt of 16 NW rows (four or eight waves, 16 rows each); the
+//   expert's pairs are gathered 16 CT at a time (CT = 1, 2 or 4) as the tokens of
+//   the LDS ring of gemm_ring_kernel (direct global -> LDS loads S - 1 super-blocks
+//   ahead)
 //   and the row tiles follow each other in one stream, so the ring stays full
 //   across them; each pair's outputs are scattered to Y[pair].
 __global__ __launch_bounds__(256) void moe_prep_kernel(const int32_t* __restrict__ ids, int n_pairs, int E,
